@@ -157,14 +157,15 @@ int kvflux_gather_paged_kv_live(const void* key_cache, const void* value_cache,
  *   bytes (no initialisation needed). Calls that share a workspace must be
  *   ordered (same stream).
  * Rows longer than one split take two launches: the split kernel and a
- * combine kernel that merges the split partials in ascending split order, so
+ * combine kernel that merges the split partials in a fixed order, so
  * results are deterministic. A split is 512 tokens; the block-size-16 kernel
  * (power-of-two block_size 1 to 256; head_size 64/128, and 256 with 16-bit
- * caches; any GQA group, as items of up to 16 heads) uses 512 to 4096 tokens
- * (pages of bs < 16 tokens: at most 256 * bs, and 256 at bs = 1), the
- * largest that leaves 8 work items per resident workgroup for num_rows rows
- * of kv_len tokens. The workspace is sized for 512-token splits (256 at
- * block_size 1), enough for either. Any group is accepted (num_rows and
+ * caches; any GQA group, as items of up to 16 heads) uses up to 4096 tokens
+ * (pages of bs < 16 tokens: at most 256 * bs, and 256 at bs = 1), and for up
+ * to 256 rows chooses the size on the device, from seq_lens, that spreads the
+ * work evenly. The least workspace accepted holds 512-token splits (256 at
+ * block_size 1); for small calls kvflux_paged_attention_workspace_size gives
+ * more, with which splits go down to 128 tokens. Any group is accepted (num_rows and
  * kv_len below 2^32, at most 65535 kv heads); shapes outside these take the
  * split kernel (head_size 64/80/96/128/256) or a generic kernel (any other
  * head_size up to 512).

@@ -177,11 +177,15 @@ struct Params {
     float* output;
     float* partial_acc;  // [rows][Hq][max_chunks][D]
     float* partial_ml;   // [rows][Hq][max_chunks][2]
-    std::uint32_t max_chunks;  // partial slots per (row, query head): ceil(kv_len / kChunk)
+    std::uint32_t max_chunks;  // partial slots per (row, query head)
     std::uint32_t row_base;  // first row of this launch slice
     std::uint32_t slice_rows;  // block-size-16 kernel: rows of this launch (at most kPlanRows)
     float scale_log2;        // log2(e) / sqrt(D)
-    std::uint32_t chunk_shift;  // block-size-16 kernel: log2(tokens per work item), 9..12
+    // Block-size-16 kernel: tokens per work item. With item_max above it the
+    // kernel picks the size from the rows' lengths, in steps of kItemStep from
+    // item_tokens to item_max.
+    std::uint32_t item_tokens;
+    std::uint32_t item_max;
     // Block-size-16 kernel: query heads per kv head (the GQA group), the
     // first of them a launch serves (0), and the head sets of a group above 8
     // (group / sub-group, each a work item of its own; 1 otherwise).
@@ -535,11 +539,17 @@ __device__ inline float row_shl(float x) {  // lane i <- lane i+kShift within a 
 //  * persistent workgroups walk a plan of (row, chunk, kv head) items built
 //    in LDS from the row lengths (exclusive prefix of chunk counts), so no
 //    workgroup is launched for an empty chunk and consecutive items read the
-//    same pages for neighbouring kv heads. A chunk is 512..4096 tokens,
-//    chosen per call (the largest that leaves enough items to balance the
-//    persistent grid): fewer, longer items mean fewer item epilogues and
-//    fewer chunk partials (4096 against 512 tokens: 1.227 against 1.37 ms
-//    for 128 rows of U[1024, 32768] tokens on MI355X). Every row's first
+//    same pages for neighbouring kv heads. A chunk is 128..4096 tokens:
+//    fewer, longer items mean fewer item epilogues and fewer chunk partials
+//    (4096 against 512 tokens: 1.227 against 1.37 ms for 128 rows of
+//    U[1024, 32768] tokens on MI355X), shorter ones fill the persistent grid
+//    evenly. The host sets the least size; up to kAdaptRows rows the kernel
+//    takes, from the lengths it plans with, the size whose longest walk is
+//    shortest: 16 rows of U[512, 8192] tokens, 28/4 heads, were 544 items of
+//    512 tokens over 512 workgroups, two rounds, and are one round of 640:
+//    35.7 -> 31.5 us; 2 rows of 40-70K tokens 69.4 -> 67.2 us with 31 instead
+//    of 137 partials a row; 4 rows of 100-1500 tokens, 128-token items over
+//    four times the workgroups, 13.3 -> 9.9 us. Every row's first
 //    chunk comes first, then the remaining chunks row by row: rows that
 //    share a prefix read it at about the same time, while it is still in
 //    the L2 of the XCD serving that kv head (that batch with a 2048-token
@@ -569,6 +579,20 @@ __device__ inline float row_shl(float x) {  // lane i <- lane i+kShift within a 
 // makes both the row-wise 16-byte writes and the transposing 8-byte reads
 // free of bank conflicts.
 constexpr int kPlanRows = 4096;
+// Item sizes the kernel chooses from where the host leaves it the choice
+// (Params::item_max): kItemSizes of them, kItemStep tokens apart, for launches
+// of up to kAdaptRows rows. kItemCost: an item's start and epilogue in tokens
+// (512 against 1024, 2048 and 4096-token items: 1.37, 1.274, 1.233 and
+// 1.222 ms for 128 rows of U[1024, 32768] tokens, so about 85; 128 also
+// weighs the partials).
+constexpr int kItemStep = 128;
+constexpr int kItemSizes = 32;
+constexpr std::uint32_t kItemCost = 128;
+constexpr std::uint32_t kAdaptRows = kThreads;
+static_assert(kThreads % kItemSizes == 0 && kItemSizes >= kWaves, "plan layout");
+// In the weight-sum place of the slot after a row's last partial (sums are
+// never negative).
+constexpr float kListEnd = -1.0f;
 
 // Column routing of the three split parts of a per-head value held by lanes
 // col < kG of each 16-lane row: set 0 gets hi in columns [0, kG), mid in
@@ -649,21 +673,9 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
     constexpr int kRowBytes = kD * 2;
     constexpr int kQPer = (kG * kD + kThreads - 1) / kThreads;
     static_assert(kRowStep * kVLoads == kBs, "V tile covers 16 tokens");
-    // Chunk of 2^chunk_shift tokens (256..4096): 16..256 tiles per item, so
-    // 4..64 (even) tiles per wavefront, whose page offsets fit one lane each
-    // (small pages: whose page slots fit one lane each).
-    const std::uint32_t chunk_shift = p.chunk_shift;
-    const std::uint32_t chunk_tokens = 1u << chunk_shift;
-    const std::uint32_t tiles = chunk_tokens / kBs;  // tiles per item
-    const int per_wave = static_cast<int>(tiles / kWaves);
-    // ceil(len / chunk_tokens) without wrapping for len near 2^32.
-    auto chunks_of = [&](std::uint32_t len) {
-        return (len >> chunk_shift) + ((len & (chunk_tokens - 1)) != 0 ? 1u : 0u);
-    };
-
     __shared__ std::uint32_t plan[kPlanRows + 1];
     __shared__ std::uint32_t lens[kPlanRows];
-    __shared__ std::uint32_t scan[kThreads];
+    __shared__ std::uint32_t scan[kItemSizes];
     // 16-bit caches: Q split in three 16-bit parts; FP32: Q as floats (two
     // 16-bit slots each). V tiles are staged for the transposing reads of the
     // 16-bit path only.
@@ -680,36 +692,80 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
 
     // ---- plan: lens[r] = row length (clamped to kv_len), plan[r] = number
     // of chunks of rows < r (a zero-length row still owns one chunk so its
-    // output is written).
-    constexpr int kPer = kPlanRows / kThreads;
-    std::uint32_t mine = 0;
-    for (int i = 0; i < kPer; ++i) {
-        const std::uint32_t r = tid * kPer + i;
+    // output is written). Thread t takes rows t * per .. of them, so a batch
+    // of up to kThreads rows reads its lengths in one round trip.
+    const std::uint32_t per = (rows + kThreads - 1) / kThreads;
+    for (std::uint32_t i = 0; i < per; ++i) {
+        const std::uint32_t r = tid * per + i;
         if (r < rows) {
             const std::uint64_t full = row_length(p, p.row_base + r);
-            const std::uint32_t len = static_cast<std::uint32_t>(full < p.kv_len ? full : p.kv_len);
-            lens[r] = len;
-            mine += len == 0 ? 1u : chunks_of(len);
+            lens[r] = static_cast<std::uint32_t>(full < p.kv_len ? full : p.kv_len);
         }
     }
-    scan[tid] = mine;
-    __syncthreads();
-    for (int off = 1; off < kThreads; off <<= 1) {
-        const std::uint32_t add = tid >= off ? scan[tid - off] : 0u;
+    // ceil(len / item) without wrapping for len near 2^32; an empty row counts one.
+    auto chunks_of = [](std::uint32_t len, std::uint32_t item) {
+        return len == 0 ? 1u : (len - 1) / item + 1;
+    };
+    // Tokens per item (a multiple of kItemStep: an even number of tiles per
+    // wavefront, at most 64, whose page offsets (small pages: page slots) fit
+    // one lane each). Where the host allows a range, every workgroup takes
+    // the size that makes the longest walk of the persistent grid shortest:
+    // ceil(items / workgroups) items of that many tokens, each with the time
+    // of kItemCost more for its start and epilogue. Lane c of a wavefront
+    // weighs candidate c, its rows split over the workgroup.
+    std::uint32_t chunk_tokens = p.item_tokens;
+    if (p.item_max > p.item_tokens) {  // uniform
+        if (tid < kItemSizes) scan[tid] = 0;
         __syncthreads();
-        scan[tid] += add;
+        const std::uint32_t c = tid % kItemSizes, size = p.item_tokens + kItemStep * c;
+        std::uint32_t n = 0;
+        if (size <= p.item_max)
+            for (std::uint32_t r = tid / kItemSizes; r < rows; r += kThreads / kItemSizes) n += chunks_of(lens[r], size);
+        atomicAdd(&scan[c], n);
         __syncthreads();
-    }
-    {
-        std::uint32_t run = scan[tid] - mine;
-        for (int i = 0; i < kPer; ++i) {
-            const std::uint32_t r = tid * kPer + i;
-            if (r < rows) {
-                plan[r] = run;
-                run += lens[r] == 0 ? 1u : chunks_of(lens[r]);
+        const std::uint32_t walk = (scan[c] * p.heads * p.q_sets + gridDim.x - 1) / gridDim.x;
+        float cost = size <= p.item_max ? static_cast<float>(walk) * static_cast<float>(size + kItemCost) : INFINITY;
+        std::uint32_t best = size;
+#pragma unroll
+        for (int x = 1; x < kItemSizes; x <<= 1) {
+            const float other_cost = __shfl_xor(cost, x);
+            const std::uint32_t other = static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(best), x));
+            if (other_cost < cost || (other_cost == cost && other > best)) {
+                cost = other_cost;
+                best = other;
             }
         }
-        if (tid == kThreads - 1) plan[rows] = scan[tid];
+        chunk_tokens = static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(best)));
+        __syncthreads();  // scan is reused
+    }
+    const std::uint32_t tiles = chunk_tokens / kBs;  // tiles per item
+    const int per_wave = static_cast<int>(tiles / kWaves);
+    // Exclusive scan of the chunk counts: within each wavefront, then over them.
+    std::uint32_t mine = 0;
+    for (std::uint32_t i = 0; i < per; ++i) {
+        const std::uint32_t r = tid * per + i;
+        if (r < rows) mine += chunks_of(lens[r], chunk_tokens);
+    }
+    std::uint32_t upto = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const std::uint32_t add = static_cast<std::uint32_t>(__shfl_up(static_cast<int>(upto), off));
+        if (lane >= off) upto += add;
+    }
+    if (lane == 63) scan[wave] = upto;
+    __syncthreads();
+    {
+        std::uint32_t run = upto - mine;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) run += w < wave ? scan[w] : 0u;
+        for (std::uint32_t i = 0; i < per; ++i) {
+            const std::uint32_t r = tid * per + i;
+            if (r < rows) {
+                plan[r] = run;
+                run += chunks_of(lens[r], chunk_tokens);
+            }
+        }
+        if (tid == kThreads - 1) plan[rows] = run;
     }
     __syncthreads();
     const std::uint32_t total = plan[rows] * p.heads * p.q_sets;
@@ -795,7 +851,7 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
             it.chunk = uniform(rx - (plan[it.row] - it.row) + 1);
         }
         const std::uint32_t len = lens[it.row];
-        const std::uint32_t begin = it.chunk << chunk_shift;
+        const std::uint32_t begin = it.chunk * chunk_tokens;
         it.ntok = uniform(len > begin ? (len - begin < chunk_tokens ? len - begin : chunk_tokens) : 0u);
         return it;
     };
@@ -806,13 +862,15 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
         const std::uint64_t* table_row =
             p.table + (p.seq_lens ? static_cast<std::uint64_t>(p.row_base) + it.row : 0) * p.width;
         if constexpr (kSmall) {
-            const std::uint32_t j = lane & ((per_wave << tps) - 1);
+            const std::uint32_t last_slot = (static_cast<std::uint32_t>(per_wave) << tps) - 1;
+            const std::uint32_t j = static_cast<std::uint32_t>(lane) < last_slot ? lane : last_slot;
             const std::uint64_t tile = static_cast<std::uint64_t>(it.chunk) * tiles + wave + kWaves * (j >> tps);
             const std::uint64_t logical = (tile << tps) + (j & ((1u << tps) - 1));
             const std::uint64_t id = table_row[logical < p.width ? logical : p.width - 1];
             return logical < p.width && id < p.num_blocks ? id * page_stride : kNoPage;
         } else {
-            const std::uint64_t tile = static_cast<std::uint64_t>(it.chunk) * tiles + wave + kWaves * (lane & (per_wave - 1));
+            const int j = lane < per_wave ? lane : per_wave - 1;
+            const std::uint64_t tile = static_cast<std::uint64_t>(it.chunk) * tiles + wave + kWaves * j;
             const std::uint64_t logical = tile >> tile_shift;
             const std::uint64_t id = table_row[logical < p.width ? logical : p.width - 1];
             const std::uint64_t in_page = (tile & ((1u << tile_shift) - 1)) * (kBs * kD);
@@ -1300,7 +1358,9 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
         }
         __syncthreads();
 
-        const bool single = lens[cur.row] <= chunk_tokens || p.max_chunks <= 1;
+        const std::uint32_t row_len = lens[cur.row];
+        const bool single = row_len <= chunk_tokens || p.max_chunks <= 1;
+        const bool last_chunk = single || cur.chunk + 1 == chunks_of(row_len, chunk_tokens);
         const std::uint32_t qh0 = cur.kvh * p.q_group + p.q_first + cur.qf;
         // The thread index is opaque here, so the epilogue's addresses are
         // formed per item rather than hoisted and held through the tile loop
@@ -1330,6 +1390,12 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
                     p.partial_ml[2 * slot + 1] = l;
                 }
             }
+            // The chunk counts follow from the item size chosen here: the
+            // slot after a row's last chunk ends its list for the combine (no
+            // partial arrays at max_chunks <= 1).
+            const std::uint32_t ends = single ? 0u : cur.chunk + 1;
+            if (d == 0 && last_chunk && p.max_chunks > 1 && ends < p.max_chunks)
+                p.partial_ml[2 * (out_row * p.max_chunks + ends) + 1] = kListEnd;
         }
         if (!has_next) break;
         __syncthreads();  // reduce, wstats and qsplit[sel] are reused
@@ -1341,72 +1407,133 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
 }
 
 // Combines the chunk partials of every (row, query head) with more than one
-// chunk. One 128-thread block per (row, query head): the chunk weights
-// exp2(m_c - m) of 128 chunks at a time go to LDS, then every thread sums its
-// dimensions over those chunks with independent loads. All sums run in
-// ascending chunk order, so results are deterministic.
-constexpr int kCombineThreads = 128;
-constexpr int kCombineMaxD = 256;  // largest head_size of the kernels that write partials
+// chunk. One 256-thread block per (row, query head): a thread holds four dims
+// (lane d4 of a group of head_dim / 4 lanes) of the chunks g, g + groups, ...
+// of its group g, with the first two chunks' loads sent out before the chunk
+// count and weights are known, and the groups are added in order through LDS.
+// Every sum has a fixed order, so results are deterministic. The work is
+// latency: the loads of all chunks are in flight at once instead of eight at a
+// time (2 rows of 137 chunks, 32 heads: 9.6 us with 128 threads walking the
+// chunks; 4.2 us now, with 31; 16 rows of 13 chunks, 28 heads: 5.3 -> 4.0 us).
+// chunk_tokens == 0: the count is the place of the first kListEnd
+// (paged_decode_bs16_kernel), else it follows from the row's length.
+// The caller's output and workspace are only known to be float-aligned.
+struct Float2 { float x, y; };
+struct Float4 { float x, y, z, w; };
+constexpr int kCombineThreads = 256;
+constexpr int kCombineWaves = kCombineThreads / 64;
 
 __global__ __launch_bounds__(kCombineThreads) void paged_attention_combine_kernel(Params p, std::uint32_t head_dim,
                                                                                    std::uint32_t chunk_tokens) {
     __shared__ float weight[kCombineThreads];
-    __shared__ float wave_max_of[kCombineThreads / 64];
+    __shared__ float wave_value[2][kCombineWaves];
+    __shared__ std::uint32_t wave_end[kCombineWaves];
+    __shared__ __attribute__((aligned(16))) float4 group_sum_of[kCombineThreads];
     const std::uint32_t row = p.row_base + blockIdx.x / p.query_heads;
     const std::uint32_t qh = blockIdx.x % p.query_heads;
-    const std::uint64_t len = row_length(p, row);
-    const std::uint64_t needed = (len + chunk_tokens - 1) / chunk_tokens;
-    const std::uint32_t nchunks =
-        needed < p.max_chunks ? static_cast<std::uint32_t>(needed) : p.max_chunks;
-    if (nchunks <= 1) return;  // uniform over the block
-    const int tid = threadIdx.x;
+    const std::uint32_t tid = threadIdx.x;
+    const int wave = tid / 64, lane = tid % 64;
     const std::uint64_t out_row = static_cast<std::uint64_t>(row) * p.query_heads + qh;
     const float* ml = p.partial_ml + out_row * p.max_chunks * 2;
     const float* acc = p.partial_acc + out_row * p.max_chunks * head_dim;
+    const std::uint32_t lanes = head_dim / 4, groups = kCombineThreads / lanes;
+    const std::uint32_t group = tid / lanes, d4 = tid % lanes;
+    const bool active = group < groups;
 
-    float m = -INFINITY;
-    for (std::uint32_t c = tid; c < nchunks; c += kCombineThreads) m = fmaxf(m, ml[2 * c]);
-    m = wave_max(m);
-    if (tid % 64 == 0) wave_max_of[tid / 64] = m;
-    __syncthreads();
-    m = fmaxf(wave_max_of[0], wave_max_of[1]);
+    // Slots past the row's chunks hold leftovers: loaded (they are within the
+    // partial arrays) and dropped.
+    auto part = [&](std::uint32_t c) {
+        const std::uint32_t safe = c < p.max_chunks ? c : p.max_chunks - 1;
+        return *reinterpret_cast<const Float4*>(acc + static_cast<std::uint64_t>(safe) * head_dim + 4 * d4);
+    };
+    const Float2 first = *reinterpret_cast<const Float2*>(ml + 2 * (tid < p.max_chunks ? tid : p.max_chunks - 1));
+    const Float4 ahead0 = part(group), ahead1 = part(group + groups);
 
-    constexpr int kDims = kCombineMaxD / kCombineThreads;
-    float o[kDims];
+    std::uint32_t nchunks;
+    if (chunk_tokens == 0) {
+        std::uint32_t end = tid < p.max_chunks && first.y == kListEnd ? tid : p.max_chunks;
+        for (std::uint32_t c = tid + kCombineThreads; c < p.max_chunks; c += kCombineThreads)
+            if (ml[2 * c + 1] == kListEnd) end = c < end ? c : end;
 #pragma unroll
-    for (int j = 0; j < kDims; ++j) o[j] = 0.0f;
-    float l = 0.0f;
+        for (int x = 1; x < 64; x <<= 1) {
+            const auto other = static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(end), x));
+            end = other < end ? other : end;
+        }
+        if (lane == 0) wave_end[wave] = end;
+        __syncthreads();
+        nchunks = wave_end[0];
+#pragma unroll
+        for (int w = 1; w < kCombineWaves; ++w) nchunks = wave_end[w] < nchunks ? wave_end[w] : nchunks;
+    } else {
+        const std::uint64_t len = row_length(p, row);
+        const std::uint64_t needed = (len + chunk_tokens - 1) / chunk_tokens;
+        nchunks = needed < p.max_chunks ? static_cast<std::uint32_t>(needed) : p.max_chunks;
+    }
+    if (nchunks == 0 || (chunk_tokens != 0 && nchunks == 1)) return;  // uniform: the row has no partials
+
+    float m = tid < nchunks ? first.x : -INFINITY;
+    for (std::uint32_t c = tid + kCombineThreads; c < nchunks; c += kCombineThreads) m = fmaxf(m, ml[2 * c]);
+    m = wave_max(m);
+    if (lane == 0) wave_value[0][wave] = m;
+    __syncthreads();
+    m = wave_value[0][0];
+#pragma unroll
+    for (int w = 1; w < kCombineWaves; ++w) m = fmaxf(m, wave_value[0][w]);
+
+    float l = 0.0f;  // this thread's chunks
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    auto add = [&](const Float4& v, float w) {
+        o.x = fmaf(v.x, w, o.x);
+        o.y = fmaf(v.y, w, o.y);
+        o.z = fmaf(v.z, w, o.z);
+        o.w = fmaf(v.w, w, o.w);
+    };
     for (std::uint32_t c0 = 0; c0 < nchunks; c0 += kCombineThreads) {
         const std::uint32_t n = nchunks - c0 < kCombineThreads ? nchunks - c0 : kCombineThreads;
-        __syncthreads();  // the previous tile's weights are no longer read
-        if (static_cast<std::uint32_t>(tid) < n) weight[tid] = exp2_shifted(ml[2 * (c0 + tid)], m);
+        if (c0 > 0) __syncthreads();  // the previous chunks' weights are no longer read
+        if (tid < n) {
+            const Float2 x = c0 == 0 ? first : *reinterpret_cast<const Float2*>(ml + 2 * (c0 + tid));
+            const float w = exp2_shifted(x.x, m);
+            weight[tid] = w;
+            l = fmaf(x.y, w, l);
+        }
         __syncthreads();
-        for (std::uint32_t c = 0; c < n; ++c) l = fmaf(ml[2 * (c0 + c) + 1], weight[c], l);
-#pragma unroll
-        for (int j = 0; j < kDims; ++j) {
-            const std::uint32_t d = tid + kCombineThreads * j;
-            if (d < head_dim) {
-                const float* src = acc + static_cast<std::uint64_t>(c0) * head_dim + d;
-                float sum = o[j];
-                std::uint32_t c = 0;
-                for (; c + 8 <= n; c += 8) {
-                    float v[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) v[u] = src[static_cast<std::uint64_t>(c + u) * head_dim];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) sum = fmaf(v[u], weight[c + u], sum);
-                }
-                for (; c < n; ++c) sum = fmaf(src[static_cast<std::uint64_t>(c) * head_dim], weight[c], sum);
-                o[j] = sum;
+        if (active) {
+            std::uint32_t c = group;
+            if (c0 == 0) {
+                if (c < n) add(ahead0, weight[c]);
+                c += groups;
+                if (c < n) add(ahead1, weight[c]);
+                c += groups;
             }
+            for (; c + 3 * groups < n; c += 4 * groups) {
+                Float4 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = part(c0 + c + u * groups);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) add(v[u], weight[c + u * groups]);
+            }
+            for (; c < n; c += groups) add(part(c0 + c), weight[c]);
         }
     }
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    l = wave_sum(l);
+    if (lane == 0) wave_value[1][wave] = l;
+    group_sum_of[tid] = o;
+    __syncthreads();
+    if (tid >= lanes) return;
+    l = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kDims; ++j) {
-        const std::uint32_t d = tid + kCombineThreads * j;
-        if (d < head_dim) p.output[out_row * head_dim + d] = o[j] * inv;
+    for (int w = 0; w < kCombineWaves; ++w) l += wave_value[1][w];
+    for (std::uint32_t g = 1; g < groups; ++g) {
+        const float4 v = group_sum_of[g * lanes + d4];
+        o.x += v.x;
+        o.y += v.y;
+        o.z += v.z;
+        o.w += v.w;
     }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    *reinterpret_cast<Float4*>(p.output + out_row * head_dim + 4 * d4) =
+        Float4{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
 }
 
 // Fallback for head sizes / group sizes without a tuned instantiation:
@@ -1534,7 +1661,8 @@ struct Plan {
     Family family = Family::Generic;
     std::uint32_t sub = 0;     // Bs16: heads per item; Split: heads per launch (divides the group)
     bool small = false;        // Bs16: pages of 1 to 8 tokens
-    std::uint32_t shift = 9;   // Bs16: log2(tokens per work item)
+    std::uint32_t item = kChunk;      // Bs16: tokens per work item, or the least of them
+    std::uint32_t item_max = kChunk;  // Bs16: above it, the kernel chooses up to this many
     unsigned grid = 0;         // Bs16: persistent grid
     std::uint64_t chunks = 0;  // partial slots per (row, query head); <= 1: no partials
     std::uint32_t rest = 0;    // Bs16: heads past the last whole set (a second launch), 0 if none
@@ -1582,11 +1710,48 @@ inline std::uint32_t log2_pow2(std::uint64_t x) {
 // Work-item tokens of the block-size-16 kernel: 2^shift with shift in
 // [9, 12] (32..256 tiles per item); pages of bs < 16 tokens cap it at
 // 4096 * bs / 16 (the item's page slots fit one per lane of a wave), down to
-// 256 tokens at bs = 1.
+// 256 tokens at bs = 1. The kernel may take a size between that and the cap
+// (Params::item_max), and small calls start at kFineItem (fine_items).
 inline std::uint32_t min_item_shift(std::uint32_t bs) { return bs >= 2 ? 9u : 8u; }
 inline std::uint32_t max_item_shift(std::uint32_t bs) { return bs >= 16 ? 12u : 8u + log2_pow2(bs); }
 
 constexpr std::uint32_t kSmallMaxGroup128 = 5;
+
+// Bytes of the partial arrays for `chunks` slots per (row, query head):
+// accumulators first, then (m, l) pairs, both 256-byte aligned.
+struct PartialLayout {
+    std::uint64_t acc_bytes = 0, total = 0;
+};
+
+PartialLayout partial_layout(std::uint64_t rows, std::uint64_t query_heads, std::uint64_t chunks,
+                             std::uint64_t head_size) {
+    PartialLayout out;
+    if (chunks <= 1) return out;
+    const std::uint64_t acc = rows * query_heads * chunks * head_size * sizeof(float);
+    const std::uint64_t ml = rows * query_heads * chunks * 2 * sizeof(float);
+    out.acc_bytes = (acc + 255) & ~std::uint64_t{255};
+    out.total = out.acc_bytes + ((ml + 255) & ~std::uint64_t{255});
+    return out;
+}
+
+// Small calls may take items down to kFineItem tokens: where 512-token items
+// would be at most kFineItems (about two per resident workgroup, so that
+// rounding to whole items leaves workgroups idle or waiting for one long
+// item) and the partials stay within kFineBytes (a quarter of the
+// no-allocation entry's scratch, so both entries plan alike). Returns the
+// bytes of partials they take, 0 where they are not used.
+constexpr std::uint32_t kFineItem = 128;
+constexpr std::uint64_t kFineItems = 1024;
+constexpr std::uint64_t kFineBytes = 8u << 20;
+static_assert(kFineBytes <= KVFLUX_NOALLOC_SCRATCH_BYTES, "both entries plan alike");
+inline std::uint64_t fine_items(std::uint64_t rows, std::uint64_t kv_len, std::uint64_t heads,
+                                std::uint64_t query_heads, std::uint64_t block_size, std::uint64_t head_size) {
+    if (!is_pow2(block_size) || block_size > 256 || (head_size != 64 && head_size != 128 && head_size != 256)) return 0;
+    if (rows > kAdaptRows || heads > kFineItems || kv_len > kFineItems * kChunk) return 0;
+    if (rows * heads * ((kv_len + kChunk - 1) / kChunk) > kFineItems || query_heads > kFineBytes) return 0;
+    const std::uint64_t bytes = partial_layout(rows, query_heads, (kv_len + kFineItem - 1) / kFineItem, head_size).total;
+    return bytes <= kFineBytes ? bytes : 0;
+}
 
 // The VALU kernels: split at head_size 64/128/256, as launches of the
 // largest power of two up to 8 (4 at 256) dividing the group, or generic.
@@ -1607,7 +1772,7 @@ inline int plan_fallback(std::uint64_t head_dim, std::uint64_t group, std::uint6
 // max_chunks: ceil(kv_len / kChunk), the partial count at 512-token items.
 template <typename E, int kD>
 int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::uint64_t max_chunks,
-               Plan* plan) {
+               std::uint64_t scratch_bytes, Plan* plan) {
     if constexpr (kD == 64 || kD == 128 || (kD == 256 && !std::is_same<E, F32>::value)) {
         // The kernel counts work items in 32 bits (at most 512-token chunks);
         // rows <= kPlanRows keeps the product below 2^51.
@@ -1677,12 +1842,19 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
                 if (wider < 8 * static_cast<std::uint64_t>(slots)) break;
                 ++shift;
             }
-            const std::uint64_t chunks = (p.kv_len + (std::uint64_t{1} << shift) - 1) >> shift;
+            // Up to kAdaptRows rows the kernel, which knows the lengths,
+            // takes the size from there on that balances the grid best.
+            std::uint32_t item = 1u << shift, item_max = item;
+            const std::uint64_t fine = fine_items(rows, p.kv_len, p.heads, p.query_heads, bs, kD);
+            if (fine > 0 && scratch_bytes >= fine && kFineItem < item) item = kFineItem;
+            const std::uint64_t chunks = (p.kv_len + item - 1) / item;
             const std::uint64_t items = rows * chunks * p.heads * sets;  // upper bound of the real count
+            if (rows <= kAdaptRows && items <= 0x7fffffffULL) item_max = 1u << max_item_shift(bs);
             plan->family = Family::Bs16;
             plan->sub = sub;
             plan->small = small;
-            plan->shift = shift;
+            plan->item = item;
+            plan->item_max = item_max;
             plan->grid = static_cast<unsigned>(items == 0 ? 1 : items < static_cast<std::uint64_t>(slots) ? items : slots);
             plan->chunks = chunks;
             plan->rest = rest;
@@ -1697,11 +1869,11 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
 
 template <typename E>
 int plan_call(const Params& p, std::uint64_t rows, std::uint64_t head_dim, std::uint64_t group,
-              std::uint64_t max_chunks, Plan* plan) {
+              std::uint64_t max_chunks, std::uint64_t scratch_bytes, Plan* plan) {
     switch (head_dim) {
-    case 64: return plan_group<E, 64>(p, rows, group, max_chunks, plan);
-    case 128: return plan_group<E, 128>(p, rows, group, max_chunks, plan);
-    case 256: return plan_group<E, 256>(p, rows, group, max_chunks, plan);
+    case 64: return plan_group<E, 64>(p, rows, group, max_chunks, scratch_bytes, plan);
+    case 128: return plan_group<E, 128>(p, rows, group, max_chunks, scratch_bytes, plan);
+    case 256: return plan_group<E, 256>(p, rows, group, max_chunks, scratch_bytes, plan);
     case 96:
     case 80: return plan_fallback(head_dim, group, max_chunks, plan);
     default: break;
@@ -1825,7 +1997,8 @@ int run_bs16(Params p, const Plan& plan, hipStream_t s) {
     p.page_tiles_shift = bs <= 16 ? 0u : log2_pow2(bs) - 4u;
     p.tile_pages_shift = bs < 16 ? 4u - log2_pow2(bs) : 0u;
     p.bs_shift = log2_pow2(bs);
-    p.chunk_shift = plan.shift;
+    p.item_tokens = plan.item;
+    p.item_max = plan.item_max;
     // One launch: a group above 8 is served as head sets of the sub-group,
     // each a work item of its own (and the heads past the last whole set, if
     // any, by a second launch).
@@ -1864,7 +2037,7 @@ int run_bs16(Params p, const Plan& plan, hipStream_t s) {
     default: status = launch_bs16<E, kD, 16>(p, plan, s); break;
     }
     if (status != KVFLUX_OK) return status;
-    if (p.max_chunks > 1) return launch_combine(p, kD, 1u << plan.shift, s);
+    if (p.max_chunks > 1) return launch_combine(p, kD, 0, s);
     return KVFLUX_OK;
 }
 
@@ -1896,29 +2069,12 @@ bool uses_split(std::uint64_t head_dim, std::uint64_t group) {
     return (head_dim == 64 || head_dim == 128 || head_dim == 256 || head_dim == 96 || head_dim == 80) && group >= 1;
 }
 
-// Bytes of the partial arrays for `chunks` slots per (row, query head):
-// accumulators first, then (m, l) pairs, both 256-byte aligned.
-struct PartialLayout {
-    std::uint64_t acc_bytes = 0, total = 0;
-};
-
-PartialLayout partial_layout(std::uint64_t rows, std::uint64_t query_heads, std::uint64_t chunks,
-                             std::uint64_t head_size) {
-    PartialLayout out;
-    if (chunks <= 1) return out;
-    const std::uint64_t acc = rows * query_heads * chunks * head_size * sizeof(float);
-    const std::uint64_t ml = rows * query_heads * chunks * 2 * sizeof(float);
-    out.acc_bytes = (acc + 255) & ~std::uint64_t{255};
-    out.total = out.acc_bytes + ((ml + 255) & ~std::uint64_t{255});
-    return out;
-}
-
 // Argument checks shared by both entry points; fills `p` and `plan`.
-// *empty = true when there is nothing to do (no rows).
+// scratch_bytes: what the caller has for the partials.
 int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks, uint64_t num_kv_heads,
             uint64_t block_size, uint64_t head_size, int dtype, const uint64_t* block_table,
             uint64_t max_blocks_per_seq, const uint64_t* seq_lens, uint64_t kv_len, uint64_t num_rows,
-            uint64_t query_heads, const float* query, float* output, Params* p, Plan* plan) {
+            uint64_t query_heads, const float* query, float* output, uint64_t scratch_bytes, Params* p, Plan* plan) {
     if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
     if (!key_cache || !value_cache || !block_table || !query || !output) {
         return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: null pointer");
@@ -1962,9 +2118,9 @@ int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks,
     p->scale_log2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(head_size)));
     int status = KVFLUX_OK;
     switch (dtype) {
-    case KVFLUX_DTYPE_BF16: status = plan_call<Bf16>(*p, num_rows, head_size, group, max_chunks, plan); break;
-    case KVFLUX_DTYPE_F16: status = plan_call<F16>(*p, num_rows, head_size, group, max_chunks, plan); break;
-    default: status = plan_call<F32>(*p, num_rows, head_size, group, max_chunks, plan); break;
+    case KVFLUX_DTYPE_BF16: status = plan_call<Bf16>(*p, num_rows, head_size, group, max_chunks, scratch_bytes, plan); break;
+    case KVFLUX_DTYPE_F16: status = plan_call<F16>(*p, num_rows, head_size, group, max_chunks, scratch_bytes, plan); break;
+    default: status = plan_call<F32>(*p, num_rows, head_size, group, max_chunks, scratch_bytes, plan); break;
     }
     if (status != KVFLUX_OK) return status;
     // The partial arrays' stride; 1 (or 0) tells the kernels that no
@@ -1987,18 +2143,19 @@ int launch_prepared(Params p, const Plan& plan, int dtype, std::uint64_t head_si
 
 using namespace kvflux_hip;
 
-extern "C" int kvflux_paged_attention_workspace_size(uint64_t num_rows, uint64_t kv_len,
-                                                     uint64_t num_kv_heads, uint64_t query_heads,
-                                                     uint64_t block_size, uint64_t head_size,
-                                                     size_t* bytes) {
-    if (!bytes) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "bytes is null");
+namespace {
+
+// The least workspace that kvflux_paged_attention accepts.
+int least_workspace(uint64_t num_rows, uint64_t kv_len,
+                    uint64_t num_kv_heads, uint64_t query_heads,
+                    uint64_t block_size, uint64_t head_size, size_t* bytes) {
     *bytes = 0;
     if (num_kv_heads == 0 || query_heads == 0 || query_heads % num_kv_heads != 0) {
         return fail(KVFLUX_ERR_INVALID_ARGUMENT, "invalid attention head counts");
     }
     if (!uses_split(head_size, query_heads / num_kv_heads)) return KVFLUX_OK;
-    // Partials of the smallest work item any kernel uses for this call:
-    // 512 tokens, 256 on pages of one token.
+    // Partials of the smallest work item that a call with any workspace may
+    // use: 512 tokens, 256 on pages of one token.
     const std::uint64_t item = block_size == 1 ? std::uint64_t{1} << min_item_shift(1) : kChunk;
     const std::uint64_t chunks = (kv_len + item - 1) / item;
     if (chunks <= 1) return KVFLUX_OK;
@@ -2008,6 +2165,20 @@ extern "C" int kvflux_paged_attention_workspace_size(uint64_t num_rows, uint64_t
         return fail(KVFLUX_ERR_OVERFLOW, "attention workspace size overflow");
     }
     *bytes = partial_layout(num_rows, query_heads, chunks, head_size).total;
+    return KVFLUX_OK;
+}
+
+} // namespace
+
+extern "C" int kvflux_paged_attention_workspace_size(uint64_t num_rows, uint64_t kv_len,
+                                                     uint64_t num_kv_heads, uint64_t query_heads,
+                                                     uint64_t block_size, uint64_t head_size,
+                                                     size_t* bytes) {
+    if (!bytes) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "bytes is null");
+    const int status = least_workspace(num_rows, kv_len, num_kv_heads, query_heads, block_size, head_size, bytes);
+    if (status != KVFLUX_OK) return status;
+    const std::uint64_t fine = fine_items(num_rows, kv_len, num_kv_heads, query_heads, block_size, head_size);
+    if (fine > *bytes) *bytes = fine;
     return KVFLUX_OK;
 }
 
@@ -2023,12 +2194,12 @@ extern "C" int kvflux_paged_attention(const void* key_cache, const void* value_c
     Plan plan;
     int status = prepare(key_cache, value_cache, num_blocks, num_kv_heads, block_size, head_size, dtype,
                          block_table, max_blocks_per_seq, seq_lens, kv_len, num_rows, query_heads, query,
-                         output, &p, &plan);
+                         output, workspace ? workspace_bytes : 0, &p, &plan);
     if (status != KVFLUX_OK) return status;
-    // The documented size (partials of 512-token items) bounds every plan.
+    // The partials of 512-token items bound every plan but the fine items',
+    // which are taken only where the workspace holds theirs.
     std::size_t need = 0;
-    status = kvflux_paged_attention_workspace_size(num_rows, kv_len, num_kv_heads, query_heads, block_size,
-                                                   head_size, &need);
+    status = least_workspace(num_rows, kv_len, num_kv_heads, query_heads, block_size, head_size, &need);
     if (status != KVFLUX_OK) return status;
     if (need > 0 && (!workspace || workspace_bytes < need)) {
         return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: workspace needs %zu bytes", need);
@@ -2101,7 +2272,7 @@ extern "C" int kvflux_paged_attention_noalloc(const void* key_cache, const void*
     Plan plan;
     int status = prepare(key_cache, value_cache, num_blocks, num_kv_heads, block_size, head_size, dtype,
                          block_table, max_blocks_per_seq, seq_lens, kv_len, num_rows, query_heads, query,
-                         output, &p, &plan);
+                         output, KVFLUX_NOALLOC_SCRATCH_BYTES, &p, &plan);
     if (status != KVFLUX_OK) return status;
     const PartialLayout layout = partial_layout(num_rows, query_heads, plan.chunks, head_size);
     if (layout.total > KVFLUX_NOALLOC_SCRATCH_BYTES) {

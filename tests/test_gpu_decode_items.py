@@ -1,0 +1,91 @@
+"""Work-item sizes of the block-size-16 decode kernel, chosen on the device
+from the row lengths: rows around multiples of the 128-token step, launches of
+one row up to one past the largest that chooses, empty rows, pages whose
+slots bound the item, a workspace of the least size (512-token items) beside
+the documented one (128-token items) and none at all where none is needed.
+Each against the oracle at 1e-5; a garbage-filled workspace must not show.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_util import DTYPES, buffer_like
+from kvflux_amd import capi, device
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5  # the exact paths' bound: FP32 sums, at most 4 more roundings per chunk merged
+
+
+def least_bytes(rows, kv_len, q_heads, block_size, head_size):
+    """Partials of 512-token items (256 on one-token pages), as documented."""
+    item = 256 if block_size == 1 else 512
+    chunks = -(-kv_len // item)
+    if chunks <= 1:
+        return 0
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    return up(rows * q_heads * chunks * head_size * 4) + up(rows * q_heads * chunks * 8)
+
+
+CASES = [
+    # dtype, kv heads, q heads, D, block size, lengths
+    ("BFloat16", 8, 32, 128, 16, [127, 128, 129, 1500]),
+    ("BFloat16", 2, 8, 128, 16, [300]),
+    ("Float16", 4, 28, 128, 16, [0, 1, 640, 641, 2047, 2048, 2049, 4000]),
+    ("Float32", 2, 8, 128, 8, [1, 255, 257, 900]),
+    ("BFloat16", 1, 4, 64, 1, [1, 256, 257, 400]),
+    ("Float16", 1, 11, 64, 64, [20000, 3]),  # a second launch for the heads past the sets
+    ("BFloat16", 2, 10, 256, 32, [513, 5000]),
+    ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(256)]),
+    ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(257)]),
+    ("Float32", 1, 1, 96, 16, [40000, 511, 512, 513]),  # the split kernel's partials, more than 64 of them
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_item_sizes(gpu, case):
+    name, H, Hq, D, bs, lens = CASES[case]
+    lib = capi.lib()
+    code, host = DTYPES[name]
+    lens = np.array(lens, np.uint64)
+    rows, max_len = len(lens), int(lens.max())
+    width = -(-max_len // bs)
+    P = width + 5
+    rng = np.random.default_rng(900 + case)
+    table = np.stack([rng.permutation(P)[:width] for _ in range(rows)]).astype(np.uint64)
+    for r in range(rows):
+        table[r, -(-int(lens[r]) // bs):] = 2**64 - 1
+    page = H * bs * D
+    kc = device.DeviceBuffer(P * page * np.dtype(host).itemsize)
+    vc = device.DeviceBuffer(P * page * np.dtype(host).itemsize)
+    device.fill_random(kc.ptr, P * page, code, 1, 40 + case)
+    device.fill_random(vc.ptr, P * page, code, 1, 80 + case)
+    q = oracle.random_elements(0, rows * Hq * D, oracle.F32, 1, 120 + case)
+    td, ld, qd = buffer_like(table.reshape(-1)), buffer_like(lens), buffer_like(q)
+    live = np.flatnonzero(lens)  # the oracle takes no empty rows
+    exp = oracle.paged_attention_rows(kc.download(host), vc.download(host), H, bs, D, code, table[live].reshape(-1),
+                                      width, lens[live], q.reshape(rows, -1)[live].reshape(-1), Hq, threads=8)
+    full = C.c_size_t(0)
+    capi.check(lib.kvflux_paged_attention_workspace_size(rows, max_len, H, Hq, bs, D, C.byref(full)))
+    least = least_bytes(rows, max_len, Hq, bs, D)
+    assert full.value >= least
+    for size in sorted({full.value, least}):
+        print(f"items case {case}: workspace {size}", flush=True)
+        ws = buffer_like(np.full(size // 4 + 64, -1.0, np.float32))  # -1: the mark that ends a row's partials
+        od = buffer_like(np.full(q.size + 8, 7.0, np.float32))
+        capi.check(lib.kvflux_paged_attention(kc.ptr, vc.ptr, P, H, bs, D, code, td.ptr, width, ld.ptr, max_len,
+                                              rows, Hq, qd.ptr, od.ptr, ws.ptr if size else None, size, None))
+        device.synchronize()
+        out = od.download(np.float32)
+        assert np.all(out[q.size:] == 7.0)
+        out = out[:q.size].reshape(rows, -1)
+        assert np.all(out[lens == 0] == 0.0)
+        assert np.abs(out[live].reshape(-1) - exp).max() < TOL
+        assert np.all(ws.download(np.float32)[size // 4:] == -1.0)
+    if least > 0:
+        status = lib.kvflux_paged_attention(kc.ptr, vc.ptr, P, H, bs, D, code, td.ptr, width, ld.ptr, max_len, rows,
+                                            Hq, qd.ptr, qd.ptr, td.ptr, least - 1, None)
+        assert status == 1  # KVFLUX_ERR_INVALID_ARGUMENT, before any launch
