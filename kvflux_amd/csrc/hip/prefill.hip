@@ -254,7 +254,12 @@ __device__ inline void set_priority() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <typename E, int kD>
+// kKs = 2: the wavefronts of a workgroup split the keys as well. Wavefronts w
+// and w + 4 hold the same rows, the first taking the first 32 keys of every
+// tile and the second the other 32, merged through LDS at the end: half the
+// rows per workgroup and half the time per tile, for launches whose
+// workgroups would leave CUs idle (prefill_choice).
+template <typename E, int kD, int kKs>
 __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams p) {
     using M = E;
     using Vec = typename M::Vec;
@@ -269,21 +274,25 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
     constexpr int kPfNt = pf_blocks<E, kD>();
     constexpr bool kExact = E::kExact;
     constexpr int kParts = kExact && !kF32 ? 3 : 1;  // 16-bit parts of Q and of the weights
-    constexpr int kBlocks = kPfWaves * kPfNt;   // 16-row blocks per workgroup
+    constexpr int kRowWaves = kPfWaves / kKs;   // wavefronts with rows of their own
+    constexpr int kHalves = 2 / kKs;            // 32-key halves of a tile per wavefront
     constexpr int kVSwz = kF32 ? 0 : kCpr / 8;  // V slot swizzle multiplier (FP32 V rows are read straight)
     constexpr float kLazy = E::kLazyLog2;
     constexpr float kWeightScale = E::kWeightScale;
     static_assert(kDma >= 1 && kTileBytes % (kPfThreads * 16) == 0, "tile split");
     static_assert(!kF32 || kD <= 128, "FP32 tiles of head_size 256 exceed the LDS");
 
-    __shared__ __attribute__((aligned(16))) std::uint16_t ktile0[kTileBytes / 2];
-    __shared__ __attribute__((aligned(16))) std::uint16_t ktile1[kTileBytes / 2];
-    __shared__ __attribute__((aligned(16))) std::uint16_t vtile0[kTileBytes / 2];
-    __shared__ __attribute__((aligned(16))) std::uint16_t vtile1[kTileBytes / 2];
+    __shared__ __attribute__((aligned(16))) std::uint16_t lds_tiles[4][kTileBytes / 2];
+    auto& ktile0 = lds_tiles[0];
+    auto& ktile1 = lds_tiles[1];
+    auto& vtile0 = lds_tiles[2];
+    auto& vtile1 = lds_tiles[3];
     __shared__ std::uint32_t pages[pf_table_max<kD>()];
 
     const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
     const int col = lane % 16, quad = lane / 16;
+    const int row_wave = wave % kRowWaves;
+    const std::uint32_t part = kKs == 1 ? 0u : __builtin_amdgcn_readfirstlane(wave / kRowWaves);  // its half of every tile
     const std::uint32_t kvh = blockIdx.x % p.heads;
     // This workgroup's sequence: the launch's one, or in a batch launch
     // sequence (blockIdx.x / heads) % num_seqs (heavy query blocks of every
@@ -346,7 +355,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 #pragma unroll
     for (int n = 0; n < kPfNt; ++n) {
         // Row 16 b + col: head (16 b + col) % G of token (16 b + col) / G.
-        const std::uint32_t r = static_cast<std::uint32_t>(16 * (wave * kPfNt + n) + col);
+        const std::uint32_t r = static_cast<std::uint32_t>(16 * (row_wave * kPfNt + n) + col);
         const std::uint32_t g = r % p.q_pass;
         const std::uint32_t token = t0 + r / p.q_pass;
         row_token[n] = token;
@@ -458,9 +467,9 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
     {
         const int s = lane % 16, r = 4 * quad + s / 4;
         const int c = (4 * (s % 4)) / 8;
-        v_read0 = r * kRowBytes + ((c ^ vswz(r)) * 16) + (s % 2) * 8;
+        v_read0 = r * kRowBytes + ((c ^ vswz(r)) * 16) + (s % 2) * 8 + 32 * part * kRowBytes;
     }
-    const std::uint32_t k_read0 = col * kRowBytes + (quad ^ kswz(col)) * 16;
+    const std::uint32_t k_read0 = col * kRowBytes + (quad ^ kswz(col)) * 16 + 32 * part * kRowBytes;
 
     pf_f32x4_t acc[kDt][kPfNt];
 #pragma unroll
@@ -481,13 +490,18 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
         nref[n] = pf_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
     bool have_ref = false;
+    // kKs = 2: a row's first keys may lie in the other wavefront's halves, so
+    // each row has its own start. -inf until the row has seen a key.
+    float lazy_of[kPfNt];
+#pragma unroll
+    for (int n = 0; n < kPfNt; ++n) lazy_of[n] = kKs == 1 ? kLazy : -INFINITY;
     const Vec ones = __builtin_bit_cast(Vec, make_uint4(M::kOnes, M::kOnes, M::kOnes, M::kOnes));
     const std::uint32_t min_limit = past + t0;
 
     auto compute_tile = [&](std::uint32_t tile, const std::uint16_t* kt, const std::uint16_t* vt) {
 #pragma unroll
-        for (int h = 0; h < kPfTile / 32; ++h) {
-            const std::uint32_t k0 = tile * kPfTile + 32 * h;
+        for (int h = 0; h < kHalves; ++h) {
+            const std::uint32_t k0 = tile * kPfTile + 32 * (h + part);
             if (k0 > last_key) break;  // uniform
             pf_f32x4_t s[2][kPfNt];
             // V^T operands of the half-tile (head_size 128): read right after
@@ -580,18 +594,20 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
             // while its row maximum is NaN enters with a zero shift for that
             // row, which changes nothing.
             float lmax[kPfNt];
-            bool grow = !have_ref;
+            bool grow = kKs == 1 && !have_ref;
 #pragma unroll
             for (int n = 0; n < kPfNt; ++n) {
                 lmax[n] = max3(max3(s[0][n][0], s[0][n][1], s[0][n][2]), max3(s[0][n][3], s[1][n][0], s[1][n][1]),
                                max3(s[1][n][2], s[1][n][3], -INFINITY));
-                grow |= lmax[n] > kLazy;
+                grow |= lmax[n] > lazy_of[n];
             }
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(grow) != 0, 0)) {
 #pragma unroll
                 for (int n = 0; n < kPfNt; ++n) {
                     const float tmax = max_across_quads(lmax[n]);
-                    const float shift = !have_ref || tmax > kLazy ? tmax : 0.0f;
+                    const bool moves = (kKs == 1 && !have_ref) || tmax > lazy_of[n];
+                    const float shift = moves ? tmax : 0.0f;
+                    if (kKs == 2 && moves) lazy_of[n] = kLazy;
                     const float alpha = __builtin_amdgcn_exp2f(fminf(-shift, 0.0f));
                     nref[n] -= shift;
                     lsum[n] *= alpha;
@@ -608,7 +624,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
                 // holds, and V dim 64g + 4col + j (one 16-byte read of the key's
                 // row per g). acc[4g + j][n][i] is then dim 64g + 16quad + 4i + j
                 // of row col.
-                const char* vrow = reinterpret_cast<const char*>(vt) + (32 * h + 4 * quad) * kRowBytes + 16 * col;
+                const char* vrow = reinterpret_cast<const char*>(vt) + (32 * (h + part) + 4 * quad) * kRowBytes + 16 * col;
                 // The tile's products are summed from zero and then added to
                 // the running accumulator (one rounding per tile): added one
                 // MFMA at a time to an accumulator dominated by one large
@@ -761,6 +777,45 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
         lds_barrier();
     }
 
+    // kKs = 2: the second halves' wavefronts hand their sums over, one row
+    // block at a time through the tile buffers (free after the loop's last
+    // barrier); the first halves' wavefronts rescale both to the higher
+    // reference point and add.
+    if constexpr (kKs == 2) {
+        constexpr int kVecs = kDt + 2;  // the accumulators, the row sums, {-reference, start}
+        static_assert(kRowWaves * kVecs * 64 * 16 <= 4 * kTileBytes, "merge buffer");
+        pf_f32x4_t* red = reinterpret_cast<pf_f32x4_t*>(&lds_tiles[0][0]) + row_wave * kVecs * 64 + lane;
+#pragma unroll
+        for (int n = 0; n < kPfNt; ++n) {
+            if (part == 1) {
+#pragma unroll
+                for (int dt = 0; dt < kDt; ++dt) red[dt * 64] = acc[dt][n];
+                red[kDt * 64] = lsum[n];
+                red[(kDt + 1) * 64] = pf_f32x4_t{nref[n][0], lazy_of[n], 0.0f, 0.0f};
+            }
+            wait_lgkm0();
+            lds_barrier();
+            if (part == 0) {
+                const pf_f32x4_t other = red[(kDt + 1) * 64];
+                const bool mine = lazy_of[n] > -INFINITY, theirs = other[1] > -INFINITY;
+                const float a = -nref[n][0], b = -other[0];
+                const float m = mine && (!theirs || a > b) ? a : b;
+                // A half without a key of the row holds zeros (factor 1).
+                const float fa = mine ? __builtin_amdgcn_exp2f(a - m) : 1.0f;
+                const float fb = theirs ? __builtin_amdgcn_exp2f(b - m) : 1.0f;
+                lsum[n] = lsum[n] * fa + red[kDt * 64] * fb;
+                nref[n][0] = -m;
+#pragma unroll
+                for (int dt = 0; dt < kDt; ++dt) acc[dt][n] = acc[dt][n] * fa + red[dt * 64] * fb;
+            }
+            if (n + 1 < kPfNt) {
+                wait_lgkm0();
+                lds_barrier();
+            }
+        }
+        if (part == 1) return;
+    }
+
 #pragma unroll
     for (int n = 0; n < kPfNt; ++n) {
         const float l = kExact ? sum_across_quads(lsum[n][0] + lsum[n][1]) : lsum[n][0];
@@ -798,54 +853,66 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 
 // Merges the key splits of every (token, query head) row: weights
 // exp2(ref_s - max ref) over the splits that saw a key, O = sum w_s O_s /
-// sum w_s l_s. One wavefront per row, lane d4 holding dims 4*d4 .. +4.
+// sum w_s l_s. D / 4 lanes per row, four dims each; four splits' loads go out
+// at once (one load at a time, behind the weight's, read the partials at
+// 2.5 TB/s: 26.6 us for 8 splits of 16384 rows).
+constexpr int kPfCombineThreads = 256;
 template <int kD>
-__global__ __launch_bounds__(256) void paged_prefill_combine_kernel(const float* __restrict__ part_o,
-                                                                    const float* __restrict__ part_ml,
-                                                                    float* __restrict__ output, std::uint64_t rows,
-                                                                    std::uint32_t splits) {
-    const std::uint64_t row = static_cast<std::uint64_t>(blockIdx.x) * 4 + threadIdx.x / 64;
-    const int lane = threadIdx.x % 64;
+__global__ __launch_bounds__(kPfCombineThreads) void paged_prefill_combine_kernel(const float* __restrict__ part_o,
+                                                                                  const float* __restrict__ part_ml,
+                                                                                  float* __restrict__ output,
+                                                                                  std::uint64_t rows,
+                                                                                  std::uint32_t splits) {
+    constexpr std::uint32_t kLanes = kD / 4, kRows = kPfCombineThreads / kLanes, kAhead = 4;
+    const std::uint64_t row = static_cast<std::uint64_t>(blockIdx.x) * kRows + threadIdx.x / kLanes;
+    const std::uint32_t d = 4 * (threadIdx.x % kLanes);
     if (row >= rows) return;
-    float m = -INFINITY;
-    for (std::uint32_t sp = 0; sp < splits; ++sp) {
-        const float2 ml = *reinterpret_cast<const float2*>(part_ml + 2 * (sp * rows + row));
-        if (ml.y > 0.0f) m = fmaxf(m, ml.x);
-    }
-    constexpr int kLanes = kD / 4;
+    float m = -INFINITY, l = 0.0f;
     float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    float l = 0.0f;
-    for (std::uint32_t sp = 0; sp < splits; ++sp) {
-        const float2 ml = *reinterpret_cast<const float2*>(part_ml + 2 * (sp * rows + row));
-        if (!(ml.y > 0.0f)) continue;  // uniform: no key of this split is visible to the row
-        const float w = __builtin_amdgcn_exp2f(ml.x - m);
-        l += w * ml.y;
-        if (lane < kLanes) {
-            const float4 x = *reinterpret_cast<const float4*>(part_o + (sp * rows + row) * kD + 4 * lane);
-            o.x += w * x.x;
-            o.y += w * x.y;
-            o.z += w * x.z;
-            o.w += w * x.w;
+    for (std::uint32_t s0 = 0; s0 < splits; s0 += kAhead) {
+        float2 ml[kAhead];
+        float4 x[kAhead];
+#pragma unroll
+        for (std::uint32_t i = 0; i < kAhead; ++i) {
+            const std::uint64_t at = (s0 + i < splits ? s0 + i : splits - 1) * rows + row;
+            ml[i] = *reinterpret_cast<const float2*>(part_ml + 2 * at);
+            x[i] = *reinterpret_cast<const float4*>(part_o + at * kD + d);
+        }
+        float top = m;
+#pragma unroll
+        for (std::uint32_t i = 0; i < kAhead; ++i)
+            if (s0 + i < splits && ml[i].y > 0.0f) top = fmaxf(top, ml[i].x);
+        const float keep = top > m ? __builtin_amdgcn_exp2f(m - top) : 1.0f;
+        l *= keep;
+        o = make_float4(o.x * keep, o.y * keep, o.z * keep, o.w * keep);
+        m = top;
+#pragma unroll
+        for (std::uint32_t i = 0; i < kAhead; ++i) {
+            if (s0 + i >= splits || !(ml[i].y > 0.0f)) continue;  // no key of this split is visible to the row
+            const float w = __builtin_amdgcn_exp2f(ml[i].x - m);
+            l += w * ml[i].y;
+            o.x += w * x[i].x;
+            o.y += w * x[i].y;
+            o.z += w * x[i].z;
+            o.w += w * x[i].w;
         }
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    if (lane < kLanes) {
-        *reinterpret_cast<float4*>(output + row * kD + 4 * lane) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
-    }
+    *reinterpret_cast<float4*>(output + row * kD + d) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
 // One launch over the heads q_first .. q_first + q_pass - 1 of every kv head.
-template <typename E, int kD>
+template <typename E, int kD, int kKs>
 int launch_prefill_pass(const PrefillParams& p, hipStream_t s) {
     PrefillParams q = p;
-    constexpr unsigned kRows = 16 * kPfWaves * pf_blocks<E, kD>();
+    constexpr unsigned kRows = 16 * (kPfWaves / kKs) * pf_blocks<E, kD>();
     q.tok = kRows / p.q_pass;
     // tq: the query tokens of the sequence, or the most of any sequence of a batch.
     q.qblocks = (p.tq + q.tok - 1) / q.tok;
     const std::uint64_t grid = static_cast<std::uint64_t>(q.qblocks) * p.heads * (p.num_seqs ? p.num_seqs : p.splits);
     if (grid > 0xffffffffULL) return fail(KVFLUX_ERR_UNSUPPORTED, "paged prefill: %llu workgroups",
                                           static_cast<unsigned long long>(grid));
-    hipLaunchKernelGGL((paged_prefill_kernel<E, kD>), dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0, s, q);
+    hipLaunchKernelGGL((paged_prefill_kernel<E, kD, kKs>), dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0, s, q);
     return launch_status("paged_prefill_kernel");
 }
 
@@ -861,7 +928,7 @@ inline std::uint32_t prefill_sub_group(std::uint32_t group, std::uint32_t rows) 
 }
 
 template <typename E, int kD>
-int launch_prefill_group(const PrefillParams& p, std::uint32_t group, hipStream_t s) {
+int launch_prefill_group(const PrefillParams& p, std::uint32_t group, int key_parts, hipStream_t s) {
     constexpr std::uint32_t kRows = 16 * kPfWaves * pf_blocks<E, kD>();
     const std::uint32_t sub = prefill_sub_group(group, kRows);
     PrefillParams q = p;
@@ -869,29 +936,32 @@ int launch_prefill_group(const PrefillParams& p, std::uint32_t group, hipStream_
     q.q_pass = sub;
     for (std::uint32_t first = 0; first < group; first += sub) {
         q.q_first = first;
-        const int st = launch_prefill_pass<E, kD>(q, s);
+        // Key parts are chosen only for groups that fit half the rows.
+        const int st = key_parts == 2 ? launch_prefill_pass<E, kD, 2>(q, s) : launch_prefill_pass<E, kD, 1>(q, s);
         if (st != KVFLUX_OK) return st;
     }
     if (p.splits > 1) {
         const std::uint64_t rows = static_cast<std::uint64_t>(p.tq) * p.query_heads;
-        hipLaunchKernelGGL(paged_prefill_combine_kernel<kD>, dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0,
-                           s, p.part_o, p.part_ml, p.output, rows, p.splits);
+        constexpr unsigned kRowsPer = kPfCombineThreads / (kD / 4);
+        hipLaunchKernelGGL(paged_prefill_combine_kernel<kD>, dim3(static_cast<unsigned>((rows + kRowsPer - 1) / kRowsPer)),
+                           dim3(kPfCombineThreads), 0, s, p.part_o, p.part_ml, p.output, rows, p.splits);
         return launch_status("paged_prefill_combine_kernel");
     }
     return KVFLUX_OK;
 }
 
 template <typename E>
-int launch_prefill_head_size(const PrefillParams& p, std::uint64_t head_size, std::uint32_t group, hipStream_t s) {
+int launch_prefill_head_size(const PrefillParams& p, std::uint64_t head_size, std::uint32_t group, int key_parts,
+                             hipStream_t s) {
     switch (head_size) {
-    case 64: return launch_prefill_group<E, 64>(p, group, s);
-    case 128: return launch_prefill_group<E, 128>(p, group, s);
+    case 64: return launch_prefill_group<E, 64>(p, group, key_parts, s);
+    case 128: return launch_prefill_group<E, 128>(p, group, key_parts, s);
     default:
         if constexpr (E::kExact) {
             return fail(KVFLUX_ERR_UNSUPPORTED, "exact paged prefill: head_size %llu",
                         static_cast<unsigned long long>(head_size));
         } else {
-            return launch_prefill_group<E, 256>(p, group, s);
+            return launch_prefill_group<E, 256>(p, group, key_parts, s);
         }
     }
 }
@@ -900,16 +970,16 @@ struct PrefillPlan {
     std::uint32_t splits;       // key splits per (query block, kv head)
     std::uint32_t split_tiles;  // 64-key tiles per split
     std::uint64_t workspace;    // bytes of partials (0 when splits == 1)
+    int key_parts;              // 2: the wavefronts of a workgroup split the keys (kKs)
 };
 
-// Key splits for a call whose launches hold fewer workgroups than about two
-// per CU (short query blocks against a long prefix, as in chunked prefill):
-// enough splits for ~512 workgroups, each of at least 4 tiles (256 keys), at
-// most 32. Partials: [splits][tq][query_heads] rows of D floats, then the
-// same rows of {reference point, weight sum}.
-inline PrefillPlan prefill_plan(std::uint64_t head_size, std::uint64_t group, std::uint64_t num_kv_heads,
-                                std::uint64_t kv_len, std::uint64_t query_tokens, std::uint64_t query_heads,
-                                bool exact = false) {
+// The most key splits a call takes, for which the workspace is sized: enough
+// for ~512 workgroups, each of at least 4 tiles (256 keys), at most 32.
+// Partials: [splits][tq][query_heads] rows of D floats, then the same rows of
+// {reference point, weight sum}.
+inline PrefillPlan prefill_most_splits(std::uint64_t head_size, std::uint64_t group, std::uint64_t num_kv_heads,
+                                       std::uint64_t kv_len, std::uint64_t query_tokens, std::uint64_t query_heads,
+                                       bool exact) {
     const std::uint64_t rows = 16 * kPfWaves * pf_blocks_for(static_cast<int>(head_size), exact);
     const std::uint64_t sub = prefill_sub_group(static_cast<std::uint32_t>(group), static_cast<std::uint32_t>(rows));
     const std::uint64_t tok = rows / sub;
@@ -922,7 +992,71 @@ inline PrefillPlan prefill_plan(std::uint64_t head_size, std::uint64_t group, st
     const std::uint64_t split_tiles = (tiles + splits - 1) / splits;
     splits = (tiles + split_tiles - 1) / split_tiles;
     const std::uint64_t ws = splits > 1 ? splits * query_tokens * query_heads * (head_size + 2) * sizeof(float) : 0;
-    return {static_cast<std::uint32_t>(splits), static_cast<std::uint32_t>(split_tiles), ws};
+    return {static_cast<std::uint32_t>(splits), static_cast<std::uint32_t>(split_tiles), ws, 1};
+}
+
+// Key splits (1 .. most_splits) and key parts (1 or 2) of a launch: the pair
+// with the shortest estimated time on 256 CUs of one resident workgroup each.
+// A workgroup takes kStart (mostly its FP32 query rows and outputs on their
+// way through memory: 256 workgroups of 64 tokens x 4 heads and one tile take
+// 17 us), then per tile the time of its MFMAs (halved with two key parts) and
+// kStep for loads and barriers; a launch takes the longest of its longest
+// workgroup and its work over all CUs, in whole rounds when the workgroups are
+// about equal (a query block behind a long prefix); splits add the partials'
+// way through memory, and two key parts have to promise a margin (more in
+// FP32, whose two 64-row workgroups load as much as one of 128).
+// Measured, BF16, 32/8 heads, D = 128, one and two key parts: 16 workgroups of
+// the latter over 1024 keys 35.4 and 25.3 us, 256 of them 40 and 32; 512 (256
+// with one) 45.8 and 73. FP32: 138 and 75, 168 and 92, 168 and 187 us. One
+// prompt of 1500 tokens, exact: no split 75.8 us (119.3 with two splits and
+// their 49 MB of partials, about 8 more with two key parts); 512 tokens behind
+// 32768: 4 splits 247 us, 8 splits 275. `share`: the part of the largest
+// case's work to expect (ragged batches, whose lengths the host has not got).
+inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32, std::uint64_t group,
+                                  std::uint64_t num_kv_heads, std::uint64_t num_seqs, std::uint64_t kv_len,
+                                  std::uint64_t query_tokens, std::uint64_t query_heads, std::uint64_t most_splits) {
+    constexpr double kCus = 256, kStart = 10.0, kStep = 0.35, kBytesPerUs = 5e6;
+    // us of a tile's MFMAs in a workgroup (8 x 4096 tokens, and 4 x 1024 in FP32)
+    const double mfma = (f32 ? 8.7 : exact ? 2.5 : 1.7) * (f32 || exact ? head_size / 128.0 : 1.0);
+    const double share = num_seqs > 1 ? 0.6 : 1.0;
+    const double margin = exact ? 1.25 : 1.05;
+    const std::uint64_t tiles = (kv_len + kPfTile - 1) / kPfTile;
+    const double past = static_cast<double>((kv_len - query_tokens) / kPfTile);
+    PrefillPlan best{1, static_cast<std::uint32_t>(tiles), 0, 1};
+    double best_time = 0;
+    for (int parts = 1; parts <= 2; ++parts) {
+        const std::uint64_t rows = 16 * (kPfWaves / parts) * pf_blocks_for(static_cast<int>(head_size), exact);
+        if (parts == 2 && group > rows) break;
+        const std::uint64_t sub = prefill_sub_group(static_cast<std::uint32_t>(group), static_cast<std::uint32_t>(rows));
+        const std::uint64_t tok = rows / sub;
+        const double blocks = static_cast<double>((query_tokens + tok - 1) / tok * num_kv_heads) * num_seqs * (group / sub);
+        const double mean_tiles = 0.5 * (past + static_cast<double>(tiles)) + 0.5;
+        const double tile_time = mfma / parts + kStep;
+        for (std::uint64_t want = 1; want <= most_splits; ++want) {
+            const std::uint64_t split_tiles = (tiles + want - 1) / want;
+            const std::uint64_t splits = (tiles + split_tiles - 1) / split_tiles;
+            if (splits != want) continue;
+            const double longest = static_cast<double>(splits == 1 ? tiles : split_tiles + 1) * tile_time + kStart;
+            const double wgs = blocks * (splits == 1 ? 1.0 : std::fmin(splits, mean_tiles / split_tiles + 1.0));
+            double time;
+            if (wgs <= kCus || past >= split_tiles) {
+                time = std::ceil(wgs / kCus) * longest;
+            } else {
+                const double even = share * (blocks * mean_tiles * tile_time + wgs * kStart) / kCus;
+                time = std::fmax(longest, even + 0.25 * longest);
+            }
+            const double partials = static_cast<double>(splits * query_tokens * query_heads * head_size) * 2 * sizeof(float);
+            if (splits > 1) time += 4.0 + partials / kBytesPerUs;
+            if (parts == 2) time *= margin;
+            if (best_time == 0 || time < best_time) {
+                best_time = time;
+                best = {static_cast<std::uint32_t>(splits), static_cast<std::uint32_t>(split_tiles), 0, parts};
+            }
+        }
+    }
+    if (best.splits > 1)
+        best.workspace = best.splits * query_tokens * query_heads * (head_size + 2) * sizeof(float);
+    return best;
 }
 
 } // namespace
@@ -978,29 +1112,34 @@ int paged_prefill(const void* key_cache, const void* value_cache, uint64_t num_b
     p.scale_log2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(head_size)));
     p.splits = 1;
     p.split_tiles = static_cast<std::uint32_t>((kv_len + kPfTile - 1) / kPfTile);
+    std::uint64_t most_splits = 1;
     if (workspace) {
-        const PrefillPlan plan = prefill_plan(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, exact);
-        if (plan.splits > 1) {
-            if (workspace_bytes < plan.workspace) {
-                return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged prefill: workspace of %llu bytes, %llu needed",
-                            static_cast<unsigned long long>(workspace_bytes),
-                            static_cast<unsigned long long>(plan.workspace));
-            }
-            p.splits = plan.splits;
-            p.split_tiles = plan.split_tiles;
-            p.part_o = static_cast<float*>(workspace);
-            p.part_ml = p.part_o + static_cast<std::uint64_t>(plan.splits) * query_tokens * query_heads * head_size;
+        const PrefillPlan most =
+            prefill_most_splits(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, exact);
+        if (workspace_bytes < most.workspace) {
+            return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged prefill: workspace of %llu bytes, %llu needed",
+                        static_cast<unsigned long long>(workspace_bytes),
+                        static_cast<unsigned long long>(most.workspace));
         }
+        most_splits = most.splits;
+    }
+    const PrefillPlan plan = prefill_choice(head_size, exact, dtype == KVFLUX_DTYPE_F32, group, num_kv_heads, 1, kv_len,
+                                            query_tokens, query_heads, most_splits);
+    if (plan.splits > 1) {
+        p.splits = plan.splits;
+        p.split_tiles = plan.split_tiles;
+        p.part_o = static_cast<float*>(workspace);
+        p.part_ml = p.part_o + static_cast<std::uint64_t>(plan.splits) * query_tokens * query_heads * head_size;
     }
     const hipStream_t s = as_stream(stream);
     const std::uint32_t g = static_cast<std::uint32_t>(group);
-    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, s);
+    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, plan.key_parts, s);
     if (exact) {
-        if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16Exact>(p, head_size, g, s);
-        return launch_prefill_head_size<PfF16Exact>(p, head_size, g, s);
+        if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16Exact>(p, head_size, g, plan.key_parts, s);
+        return launch_prefill_head_size<PfF16Exact>(p, head_size, g, plan.key_parts, s);
     }
-    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, s);
-    return launch_prefill_head_size<PfF16>(p, head_size, g, s);
+    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, plan.key_parts, s);
+    return launch_prefill_head_size<PfF16>(p, head_size, g, plan.key_parts, s);
 }
 
 } // namespace
@@ -1029,9 +1168,9 @@ extern "C" int kvflux_paged_prefill_workspace_size(uint64_t num_kv_heads, uint64
     // fewer workgroups and plan more key splits.
     const std::uint64_t group = query_heads / num_kv_heads;
     const std::uint64_t rounded =
-        prefill_plan(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, false).workspace;
+        prefill_most_splits(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, false).workspace;
     const std::uint64_t exact =
-        head_size == 256 ? 0 : prefill_plan(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, true).workspace;
+        head_size == 256 ? 0 : prefill_most_splits(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, true).workspace;
     *bytes = static_cast<size_t>(rounded > exact ? rounded : exact);
     return KVFLUX_OK;
 }
@@ -1109,7 +1248,10 @@ extern "C" int kvflux_paged_prefill_batch(const void* key_cache, const void* val
     p.seq_q_offsets = query_offsets;
     const hipStream_t s = as_stream(stream);
     const std::uint32_t g = static_cast<std::uint32_t>(query_heads / num_kv_heads);
-    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, s);
-    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, s);
-    return launch_prefill_head_size<PfF16>(p, head_size, g, s);
+    const bool f32 = dtype == KVFLUX_DTYPE_F32;
+    const PrefillPlan plan = prefill_choice(head_size, f32, f32, g, num_kv_heads, num_seqs, max_kv_len,
+                                            max_query_tokens, query_heads, 1);
+    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, plan.key_parts, s);
+    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, plan.key_parts, s);
+    return launch_prefill_head_size<PfF16>(p, head_size, g, plan.key_parts, s);
 }
