@@ -1,5 +1,5 @@
 // Causal paged prefill on MFMA (gfx950): BF16/FP16 caches, head_size 64/128/256,
-// and FP32 caches, head_size 64/128 (v_mfma_f32_16x16x4_f32, see PfF32).
+// and FP32 caches, head_size 64/128 (paged_prefill_f32_kernel).
 //
 // One workgroup (8 wavefronts, two per SIMD) owns one kv head and 16 * R rows
 // (R = 8 * pf_blocks row blocks of 16: 32 at head_size 64, 16 at 128, 8 at
@@ -58,7 +58,6 @@ struct PfBf16 {
     static constexpr float kWeightScale = 1.0f;
     static constexpr float kLazyLog2 = 8.0f;
     static constexpr bool kExact = false;
-    static constexpr bool kF32 = false;
     static constexpr std::uint32_t kOnes = 0x3f803f80u;  // two 1.0
     __device__ static std::uint32_t pack(float a, float b) {
         return __builtin_bit_cast(std::uint32_t, __builtin_convertvector(pf_f32x2_t{a, b}, pf_bf16x2_t));
@@ -81,7 +80,6 @@ struct PfF16 {
     static constexpr float kWeightScale = 1.0f;
     static constexpr float kLazyLog2 = 8.0f;
     static constexpr bool kExact = false;
-    static constexpr bool kF32 = false;
     static constexpr std::uint32_t kOnes = 0x3c003c00u;  // two 1.0
     __device__ static std::uint32_t pack(float a, float b) {
         return __builtin_bit_cast(std::uint32_t, __builtin_convertvector(pf_f32x2_t{a, b}, pf_f16x2_t));
@@ -118,20 +116,9 @@ struct PfF16Exact : PfF16 {
     static constexpr float kWeightScale = 32768.0f;
     static constexpr float kLazyLog2 = 0.0f;
 };
-// FP32 caches: K, V, Q and the weights enter v_mfma_f32_16x16x4_f32 as they
-// are (exact products, FP32 accumulation), with the exact variants' FP32 row
-// sums and one row block per wavefront. Vec only sizes the 16-bit operand
-// arrays, which this policy leaves unused.
+// FP32 caches (paged_prefill_f32_kernel): rows per workgroup as in the exact variants.
 struct PfF32 {
-    using Vec = pf_bf16x8_t;
-    static constexpr float kWeightScale = 1.0f;
-    static constexpr float kLazyLog2 = 8.0f;
     static constexpr bool kExact = true;
-    static constexpr bool kF32 = true;
-    static constexpr std::uint32_t kOnes = 0;
-    __device__ static pf_f32x4_t mma4(float a, float b, const pf_f32x4_t& c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
 };
 
 // NaN-propagating maximum of three (one v_maximum3_f32).
@@ -254,6 +241,57 @@ __device__ inline void set_priority() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// What a workgroup works on: its sequence (the launch's one, or in a batch
+// launch sequence (blockIdx.x / heads) % num_seqs, heavy query blocks of every
+// sequence first), query block and key split. All values wave-uniform.
+struct PfShare {
+    std::uint32_t split, kv_len, tq, table_len;
+    const std::uint64_t* table;
+    const float* query;
+    float* output;
+    std::uint32_t t0, t_end;  // query tokens
+    std::uint32_t past, last_key, ntiles;
+    // This split's tiles. The split holding the tile of the first row's
+    // position runs to the last tile and later splits are empty, so every
+    // split a workgroup runs starts at a key all its rows see (each row then
+    // sets its reference point on the first half-tile).
+    std::uint32_t tile_begin, tile_end;
+    bool idle;  // no rows
+};
+template <int kD>
+__device__ inline PfShare pf_share(const PrefillParams& p) {
+    PfShare w{0, p.kv_len, p.tq, p.table_len, p.table, p.query, p.output, 0, 0, 0, 0, 0, 0, 0, false};
+    std::uint32_t qb;
+    if (p.num_seqs == 0) {
+        w.split = (blockIdx.x / p.heads) % p.splits;
+        qb = p.qblocks - 1 - blockIdx.x / p.heads / p.splits;
+    } else {
+        const std::uint32_t seq = (blockIdx.x / p.heads) % p.num_seqs;
+        qb = p.qblocks - 1 - blockIdx.x / p.heads / p.num_seqs;
+        const std::uint64_t kvl = p.seq_kv_lens[seq], ql = p.seq_q_lens[seq], q0 = p.seq_q_offsets[seq];
+        w.kv_len = static_cast<std::uint32_t>(kvl < p.kv_len ? kvl : p.kv_len);
+        w.tq = static_cast<std::uint32_t>(ql < w.kv_len ? ql : w.kv_len);
+        w.table = p.table + static_cast<std::uint64_t>(seq) * p.table_len;
+        w.query = p.query + q0 * p.query_heads * kD;
+        w.output = p.output + q0 * p.query_heads * kD;
+        if (w.tq == 0 || static_cast<std::uint64_t>(qb) * p.tok >= w.tq) {
+            w.idle = true;
+            return w;
+        }
+    }
+    w.t0 = qb * p.tok;
+    w.t_end = w.t0 + p.tok < w.tq ? w.t0 + p.tok : w.tq;
+    w.past = w.kv_len - w.tq;
+    w.last_key = w.past + w.t_end - 1;
+    w.ntiles = w.last_key / kPfTile + 1;
+    const std::uint32_t first_row_tile = (w.past + w.t0) / kPfTile;
+    w.tile_begin = w.split * p.split_tiles;
+    w.tile_end = w.tile_begin + p.split_tiles;
+    if (w.tile_end > first_row_tile) w.tile_end = w.ntiles;
+    if (w.tile_begin > first_row_tile) w.tile_begin = w.tile_end;
+    return w;
+}
+
 // kKs = 2: the wavefronts of a workgroup split the keys as well. Wavefronts w
 // and w + 4 hold the same rows, the first taking the first 32 keys of every
 // tile and the second the other 32, merged through LDS at the end: half the
@@ -263,24 +301,22 @@ template <typename E, int kD, int kKs>
 __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams p) {
     using M = E;
     using Vec = typename M::Vec;
-    constexpr bool kF32 = E::kF32;
-    constexpr int kSteps = kD / 32;            // K-dim steps of S^T (16-bit)
-    constexpr int kQuads = kD / 16;            // 16-dim chunks of S^T (FP32: four MFMAs each)
+    constexpr int kSteps = kD / 32;            // K-dim steps of S^T
+    constexpr int kQuads = kD / 16;            // 16-dim chunks of Q
     constexpr int kDt = kD / 16;               // dim blocks of O^T
-    constexpr int kRowBytes = kD * (kF32 ? 4 : 2);
+    constexpr int kRowBytes = kD * 2;
     constexpr int kCpr = kRowBytes / 16;       // 16-byte chunks per key row
     constexpr int kTileBytes = kPfTile * kRowBytes;
     constexpr int kDma = kTileBytes / (kPfThreads * 16);  // tile loads per thread per cache
     constexpr int kPfNt = pf_blocks<E, kD>();
     constexpr bool kExact = E::kExact;
-    constexpr int kParts = kExact && !kF32 ? 3 : 1;  // 16-bit parts of Q and of the weights
+    constexpr int kParts = kExact ? 3 : 1;  // 16-bit parts of Q and of the weights
     constexpr int kRowWaves = kPfWaves / kKs;   // wavefronts with rows of their own
     constexpr int kHalves = 2 / kKs;            // 32-key halves of a tile per wavefront
-    constexpr int kVSwz = kF32 ? 0 : kCpr / 8;  // V slot swizzle multiplier (FP32 V rows are read straight)
+    constexpr int kVSwz = kCpr / 8;  // V slot swizzle multiplier
     constexpr float kLazy = E::kLazyLog2;
     constexpr float kWeightScale = E::kWeightScale;
     static_assert(kDma >= 1 && kTileBytes % (kPfThreads * 16) == 0, "tile split");
-    static_assert(!kF32 || kD <= 128, "FP32 tiles of head_size 256 exceed the LDS");
 
     __shared__ __attribute__((aligned(16))) std::uint16_t lds_tiles[4][kTileBytes / 2];
     auto& ktile0 = lds_tiles[0];
@@ -294,41 +330,14 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
     const int row_wave = wave % kRowWaves;
     const std::uint32_t part = kKs == 1 ? 0u : __builtin_amdgcn_readfirstlane(wave / kRowWaves);  // its half of every tile
     const std::uint32_t kvh = blockIdx.x % p.heads;
-    // This workgroup's sequence: the launch's one, or in a batch launch
-    // sequence (blockIdx.x / heads) % num_seqs (heavy query blocks of every
-    // sequence first). All values wave-uniform.
-    std::uint32_t split = 0, qb = 0, kv_len = p.kv_len, tq = p.tq, table_len = p.table_len;
-    const std::uint64_t* table = p.table;
-    const float* query = p.query;
-    float* output = p.output;
-    if (p.num_seqs == 0) {
-        split = (blockIdx.x / p.heads) % p.splits;
-        qb = p.qblocks - 1 - blockIdx.x / p.heads / p.splits;
-    } else {
-        const std::uint32_t seq = (blockIdx.x / p.heads) % p.num_seqs;
-        qb = p.qblocks - 1 - blockIdx.x / p.heads / p.num_seqs;
-        const std::uint64_t kvl = p.seq_kv_lens[seq], ql = p.seq_q_lens[seq], q0 = p.seq_q_offsets[seq];
-        kv_len = static_cast<std::uint32_t>(kvl < p.kv_len ? kvl : p.kv_len);
-        tq = static_cast<std::uint32_t>(ql < kv_len ? ql : kv_len);
-        table = p.table + static_cast<std::uint64_t>(seq) * p.table_len;
-        query = p.query + q0 * p.query_heads * kD;
-        output = p.output + q0 * p.query_heads * kD;
-        if (tq == 0 || static_cast<std::uint64_t>(qb) * p.tok >= tq) return;  // uniform
-    }
-    const std::uint32_t t0 = qb * p.tok;
-    const std::uint32_t t_end = t0 + p.tok < tq ? t0 + p.tok : tq;
-    const std::uint32_t past = kv_len - tq;
-    const std::uint32_t last_key = past + t_end - 1;
-    const std::uint32_t ntiles = last_key / kPfTile + 1;
-    // This split's tiles [tile_begin, tile_end). The split holding the tile of
-    // the first row's position runs to the last tile and later splits are
-    // empty, so every split a workgroup runs starts at a key all its rows see
-    // (each row then sets its reference point on the first half-tile).
-    const std::uint32_t first_row_tile = (past + t0) / kPfTile;
-    std::uint32_t tile_begin = split * p.split_tiles;
-    std::uint32_t tile_end = tile_begin + p.split_tiles;
-    if (tile_end > first_row_tile) tile_end = ntiles;
-    if (tile_begin > first_row_tile) tile_begin = tile_end;
+    const PfShare share = pf_share<kD>(p);
+    if (share.idle) return;  // uniform
+    const std::uint32_t split = share.split, kv_len = share.kv_len, tq = share.tq, table_len = share.table_len;
+    const std::uint32_t t0 = share.t0, t_end = share.t_end, past = share.past, last_key = share.last_key;
+    const std::uint32_t ntiles = share.ntiles, tile_begin = share.tile_begin, tile_end = share.tile_end;
+    const std::uint64_t* const table = share.table;
+    const float* const query = share.query;
+    float* const output = share.output;
     const std::uint32_t npages = ((ntiles * kPfTile - 1) >> p.bs_shift) + 1;
     // Key k of the sequence lies in page k >> bs_shift, row k & (bs - 1).
     // The page list holds a window of kWin pages (whole tiles) at a time: page
@@ -348,8 +357,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
     };
     // The query rows' loads go out before the page list's, so the two round
     // trips overlap; the rows are rounded to the cache dtype after.
-    // 16-bit caches: float4 pairs 2kk, 2kk + 1 are dims 32kk + 8quad .. +8 of
-    // the row; FP32: float4 c is dims 16c + 4quad .. +4.
+    // float4 pairs 2kk, 2kk + 1 are dims 32kk + 8quad .. +8 of the row.
     float4 qraw[kPfNt][kQuads];
     std::uint32_t row_token[kPfNt], row_head[kPfNt];
 #pragma unroll
@@ -365,43 +373,33 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
             query + (static_cast<std::uint64_t>(tq_safe) * p.query_heads + kvh * p.q_group + p.q_first + g) * kD;
 #pragma unroll
         for (int c = 0; c < kQuads; ++c) {
-            const int off = kF32 ? 16 * c + 4 * quad : 32 * (c / 2) + 8 * quad + 4 * (c % 2);
+            const int off = 32 * (c / 2) + 8 * quad + 4 * (c % 2);
             qraw[n][c] = *reinterpret_cast<const float4*>(src + off);
         }
     }
     stage(first_page(tile_begin & ~win_mask));
-    // FP32: Q * scale as it is, lane (quad, col) dims 16c + 4quad + j in qf[n][c][j].
-    pf_f32x4_t qf[kF32 ? kPfNt : 1][kF32 ? kQuads : 1];
-    Vec qb_op[kParts][kF32 ? 1 : kPfNt][kF32 ? 1 : kSteps];
+    Vec qb_op[kParts][kPfNt][kSteps];
 #pragma unroll
     for (int n = 0; n < kPfNt; ++n) {
-        if constexpr (kF32) {
 #pragma unroll
-            for (int c = 0; c < kQuads; ++c) {
-                const float4 v = qraw[n][c];
-                qf[n][c] = pf_f32x4_t{v.x, v.y, v.z, v.w} * p.scale_log2;
-            }
-        } else {
+        for (int kk = 0; kk < kSteps; ++kk) {
+            const float4 lo = qraw[n][2 * kk], hi = qraw[n][2 * kk + 1];
+            const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            std::uint32_t w[kParts][4];
 #pragma unroll
-            for (int kk = 0; kk < kSteps; ++kk) {
-                const float4 lo = qraw[n][2 * kk], hi = qraw[n][2 * kk + 1];
-                const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                std::uint32_t w[kParts][4];
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (kExact) {
+                    std::uint32_t parts[3];
+                    M::split3(v[2 * e] * p.scale_log2, v[2 * e + 1] * p.scale_log2, parts);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if constexpr (kExact) {
-                        std::uint32_t parts[3];
-                        M::split3(v[2 * e] * p.scale_log2, v[2 * e + 1] * p.scale_log2, parts);
-#pragma unroll
-                        for (int k = 0; k < kParts; ++k) w[k][e] = parts[k];
-                    } else {
-                        w[0][e] = M::pack(v[2 * e] * p.scale_log2, v[2 * e + 1] * p.scale_log2);
-                    }
+                    for (int k = 0; k < kParts; ++k) w[k][e] = parts[k];
+                } else {
+                    w[0][e] = M::pack(v[2 * e] * p.scale_log2, v[2 * e + 1] * p.scale_log2);
                 }
-#pragma unroll
-                for (int k = 0; k < kParts; ++k)
-                    qb_op[k][n][kk] = __builtin_bit_cast(Vec, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
             }
+#pragma unroll
+            for (int k = 0; k < kParts; ++k)
+                qb_op[k][n][kk] = __builtin_bit_cast(Vec, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
         }
     }
     __syncthreads();  // pages[] ready (the query loads are complete as well)
@@ -518,63 +516,36 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
                     __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4_t*)(vbase + off + 16 * kRowBytes));
                 return __builtin_bit_cast(Vec, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
             };
-            constexpr bool kEarlyV = kD == 128 && !kF32;
+            constexpr bool kEarlyV = kD == 128;
             Vec vop[kEarlyV ? kDt : 1];
             set_priority<1>();
-            if constexpr (kF32) {
-                // MFMA (c, j) takes, in lane (quad, col), dim 16c + 4quad + j of
-                // key col (K, one 16-byte read per c) and of row col (Q); the
-                // dim order does not change the sum.
+            Vec a[kSteps][2];
+#pragma unroll
+            for (int kk = 0; kk < kSteps; ++kk)
+#pragma unroll
+                for (int kt2 = 0; kt2 < 2; ++kt2)
+                    a[kk][kt2] = __builtin_bit_cast(
+                        Vec, *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(kt) +
+                                                             (32 * h + 16 * kt2) * kRowBytes + (k_read0 ^ (kk << 6))));
+#pragma unroll
+            for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+                for (int n = 0; n < kPfNt; ++n) s[kt2][n] = nref[n];
+#pragma unroll
+            for (int kk = 0; kk < kSteps; ++kk)
 #pragma unroll
                 for (int kt2 = 0; kt2 < 2; ++kt2)
 #pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) s[kt2][n] = nref[n];
+                    for (int n = 0; n < kPfNt; ++n)
 #pragma unroll
-                for (int c = 0; c < kQuads; ++c) {
-                    float4 a[2];
+                        for (int k = 0; k < kParts; ++k) s[kt2][n] = M::mma(a[kk][kt2], qb_op[k][n][kk], s[kt2][n]);
+            if constexpr (kEarlyV) {
 #pragma unroll
-                    for (int kt2 = 0; kt2 < 2; ++kt2)
-                        a[kt2] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(kt) +
-                                                                  (32 * h + 16 * kt2) * kRowBytes + (k_read0 ^ (c << 6)));
-#pragma unroll
-                    for (int kt2 = 0; kt2 < 2; ++kt2)
-#pragma unroll
-                        for (int n = 0; n < kPfNt; ++n) {
-                            s[kt2][n] = M::mma4(a[kt2].x, qf[n][c][0], s[kt2][n]);
-                            s[kt2][n] = M::mma4(a[kt2].y, qf[n][c][1], s[kt2][n]);
-                            s[kt2][n] = M::mma4(a[kt2].z, qf[n][c][2], s[kt2][n]);
-                            s[kt2][n] = M::mma4(a[kt2].w, qf[n][c][3], s[kt2][n]);
-                        }
-                }
-            } else {
-                Vec a[kSteps][2];
-#pragma unroll
-                for (int kk = 0; kk < kSteps; ++kk)
-#pragma unroll
-                    for (int kt2 = 0; kt2 < 2; ++kt2)
-                        a[kk][kt2] = __builtin_bit_cast(
-                            Vec, *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(kt) +
-                                                                 (32 * h + 16 * kt2) * kRowBytes + (k_read0 ^ (kk << 6))));
-#pragma unroll
-                for (int kt2 = 0; kt2 < 2; ++kt2)
-#pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) s[kt2][n] = nref[n];
-#pragma unroll
-                for (int kk = 0; kk < kSteps; ++kk)
-#pragma unroll
-                    for (int kt2 = 0; kt2 < 2; ++kt2)
-#pragma unroll
-                        for (int n = 0; n < kPfNt; ++n)
-#pragma unroll
-                            for (int k = 0; k < kParts; ++k) s[kt2][n] = M::mma(a[kk][kt2], qb_op[k][n][kk], s[kt2][n]);
-                if constexpr (kEarlyV) {
-#pragma unroll
-                    for (int dt = 0; dt < kDt; ++dt) vop[dt] = read_v(dt);
-                    // The K reads first, then the MFMAs, then the V reads.
-                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kSteps, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2 * kSteps * kPfNt * kParts, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kDt, 0);
-                }
+                for (int dt = 0; dt < kDt; ++dt) vop[dt] = read_v(dt);
+                // The K reads first, then the MFMAs, then the V reads.
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * kSteps, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 2 * kSteps * kPfNt * kParts, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * kDt, 0);
             }
             set_priority<0>();
             if (k0 + 31 > min_limit) {
@@ -618,112 +589,61 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
                 }
                 have_ref = true;
             }
-            if constexpr (kF32) {
-                // O^T += V^T P^T over keys: MFMA (kt2, r, g, j) takes key
-                // 16kt2 + 4quad + r in lane (quad, col), the weight the lane
-                // holds, and V dim 64g + 4col + j (one 16-byte read of the key's
-                // row per g). acc[4g + j][n][i] is then dim 64g + 16quad + 4i + j
-                // of row col.
-                const char* vrow = reinterpret_cast<const char*>(vt) + (32 * (h + part) + 4 * quad) * kRowBytes + 16 * col;
-                // The tile's products are summed from zero and then added to
-                // the running accumulator (one rounding per tile): added one
-                // MFMA at a time to an accumulator dominated by one large
-                // weight, small weights lose bits in the same direction at
-                // every step (measured: 2.8e-5 on a row of one dominant key
-                // and 4095 keys 2^-25 below it).
-                pf_f32x4_t tpart[kD / 16][kPfNt];
+            Vec pb[kParts][kPfNt];
 #pragma unroll
-                for (int i = 0; i < kD / 16; ++i)
+            for (int n = 0; n < kPfNt; ++n) {
+                float pr[8];
 #pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) tpart[i][n] = pf_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int kt2 = 0; kt2 < 2; ++kt2)
 #pragma unroll
-                for (int kt2 = 0; kt2 < 2; ++kt2) {
-                    float pr[kPfNt][4];
+                    for (int r = 0; r < 4; ++r) pr[4 * kt2 + r] = __builtin_amdgcn_exp2f(s[kt2][n][r]);
+                std::uint32_t w[kParts][4];
+                if constexpr (kExact) {
+                    float hi = lsum[n][0], lo = lsum[n][1];  // [1]: the sum's low word
+                    two_sum_add(hi, lo, ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7])));
+                    lsum[n][0] = hi;
+                    lsum[n][1] = lo;
 #pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) {
+                    for (int j = 0; j < 4; ++j) {
+                        std::uint32_t parts[3];
+                        M::split3(pr[2 * j] * kWeightScale, pr[2 * j + 1] * kWeightScale, parts);
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) pr[n][r] = __builtin_amdgcn_exp2f(s[kt2][n][r]);
-                        float hi = lsum[n][0], lo = lsum[n][1];  // [1]: the sum's low word
-                        two_sum_add(hi, lo, (pr[n][0] + pr[n][1]) + (pr[n][2] + pr[n][3]));
-                        lsum[n][0] = hi;
-                        lsum[n][1] = lo;
+                        for (int k = 0; k < kParts; ++k) w[k][j] = parts[k];
                     }
+                } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int g = 0; g < kD / 64; ++g) {
-                            const float4 v =
-                                *reinterpret_cast<const float4*>(vrow + (16 * kt2 + r) * kRowBytes + 256 * g);
-#pragma unroll
-                            for (int n = 0; n < kPfNt; ++n) {
-                                tpart[4 * g][n] = M::mma4(v.x, pr[n][r], tpart[4 * g][n]);
-                                tpart[4 * g + 1][n] = M::mma4(v.y, pr[n][r], tpart[4 * g + 1][n]);
-                                tpart[4 * g + 2][n] = M::mma4(v.z, pr[n][r], tpart[4 * g + 2][n]);
-                                tpart[4 * g + 3][n] = M::mma4(v.w, pr[n][r], tpart[4 * g + 3][n]);
-                            }
-                        }
+                    for (int j = 0; j < 4; ++j) w[0][j] = M::pack(pr[2 * j], pr[2 * j + 1]);
                 }
 #pragma unroll
-                for (int i = 0; i < kD / 16; ++i)
+                for (int k = 0; k < kParts; ++k) pb[k][n] = __builtin_bit_cast(Vec, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
+            }
 #pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) acc[i][n] += tpart[i][n];
-            } else {
-                Vec pb[kParts][kPfNt];
+            for (int dt = 0; dt < kDt; ++dt) {
+                Vec a;
+                if constexpr (kEarlyV) {
+                    a = vop[dt];
+                } else {
+                    a = read_v(dt);
+                }
 #pragma unroll
                 for (int n = 0; n < kPfNt; ++n) {
-                    float pr[8];
-#pragma unroll
-                    for (int kt2 = 0; kt2 < 2; ++kt2)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) pr[4 * kt2 + r] = __builtin_amdgcn_exp2f(s[kt2][n][r]);
-                    std::uint32_t w[kParts][4];
                     if constexpr (kExact) {
-                        float hi = lsum[n][0], lo = lsum[n][1];  // [1]: the sum's low word
-                        two_sum_add(hi, lo, ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7])));
-                        lsum[n][0] = hi;
-                        lsum[n][1] = lo;
+                        // The tile's three parts summed from zero, then
+                        // one rounding into the running accumulator (see
+                        // the FP32 kernel below).
+                        pf_f32x4_t t = M::mma(a, pb[0][n], pf_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            std::uint32_t parts[3];
-                            M::split3(pr[2 * j] * kWeightScale, pr[2 * j + 1] * kWeightScale, parts);
-#pragma unroll
-                            for (int k = 0; k < kParts; ++k) w[k][j] = parts[k];
-                        }
+                        for (int k = 1; k < kParts; ++k) t = M::mma(a, pb[k][n], t);
+                        acc[dt][n] += t;
                     } else {
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) w[0][j] = M::pack(pr[2 * j], pr[2 * j + 1]);
-                    }
-#pragma unroll
-                    for (int k = 0; k < kParts; ++k) pb[k][n] = __builtin_bit_cast(Vec, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
-                }
-#pragma unroll
-                for (int dt = 0; dt < kDt; ++dt) {
-                    Vec a;
-                    if constexpr (kEarlyV) {
-                        a = vop[dt];
-                    } else {
-                        a = read_v(dt);
-                    }
-#pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) {
-                        if constexpr (kExact) {
-                            // The tile's three parts summed from zero, then
-                            // one rounding into the running accumulator (see
-                            // the FP32 path above).
-                            pf_f32x4_t t = M::mma(a, pb[0][n], pf_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-                            for (int k = 1; k < kParts; ++k) t = M::mma(a, pb[k][n], t);
-                            acc[dt][n] += t;
-                        } else {
-#pragma unroll
-                            for (int k = 0; k < kParts; ++k) acc[dt][n] = M::mma(a, pb[k][n], acc[dt][n]);
-                        }
+                        for (int k = 0; k < kParts; ++k) acc[dt][n] = M::mma(a, pb[k][n], acc[dt][n]);
                     }
                 }
-                if constexpr (!kExact) {
+            }
+            if constexpr (!kExact) {
 #pragma unroll
-                    for (int n = 0; n < kPfNt; ++n) lsum[n] = M::mma(ones, pb[0][n], lsum[n]);
-                }
+                for (int n = 0; n < kPfNt; ++n) lsum[n] = M::mma(ones, pb[0][n], lsum[n]);
             }
         }
     };
@@ -830,24 +750,376 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
             const std::uint64_t prow = static_cast<std::uint64_t>(split) * tq * p.query_heads + row;
             float* dst = whole ? output + row * kD : p.part_o + prow * kD;
             const float sc = (whole ? inv : 1.0f) * (1.0f / kWeightScale);  // kWeightScale: a power of two
-            if constexpr (kF32) {
 #pragma unroll
-                for (int g = 0; g < kD / 64; ++g)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        *reinterpret_cast<float4*>(dst + 64 * g + 16 * quad + 4 * i) =
-                            make_float4(acc[4 * g][n][i] * sc, acc[4 * g + 1][n][i] * sc, acc[4 * g + 2][n][i] * sc,
-                                        acc[4 * g + 3][n][i] * sc);
-            } else {
-#pragma unroll
-                for (int dt = 0; dt < kDt; ++dt) {
-                    *reinterpret_cast<float4*>(dst + 16 * dt + 4 * quad) =
-                        make_float4(acc[dt][n][0] * sc, acc[dt][n][1] * sc, acc[dt][n][2] * sc, acc[dt][n][3] * sc);
-                }
+            for (int dt = 0; dt < kDt; ++dt) {
+                *reinterpret_cast<float4*>(dst + 16 * dt + 4 * quad) =
+                    make_float4(acc[dt][n][0] * sc, acc[dt][n][1] * sc, acc[dt][n][2] * sc, acc[dt][n][3] * sc);
             }
             // An empty split leaves l = 0; the combine skips it.
             if (!whole && quad == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(-nref[n][0], l);
         }
+    }
+}
+
+// FP32 caches: the exact variant's plan with K and V in three BF16 parts as
+// well. v_mfma_f32_16x16x4_f32 runs at a sixteenth of the BF16 rate, and a
+// kernel on it is bound by it (124 of 157 TFLOP/s, 8.4 us per 128 rows x 64
+// keys); with x = hi + mid + lo (8 bits each, exact) a product is the six part
+// products down to 2^-18 of it, the three dropped ones being under 2^-26, less
+// than half the rounding of one FP32 product: six BF16 MFMAs for 32 dims in
+// place of eight FP32 ones of twice the time each.
+//  * The parts of a half-tile (32 keys) are made once per workgroup, on the
+//    way from global memory (registers, one half ahead of its use) to LDS, and
+//    are double-buffered there (96 KiB at head_size 128): one barrier per half,
+//    and a wavefront's conversions run beside the other's MFMAs.
+//  * The smaller part products are summed apart from the large ones and added
+//    last, in QK^T and in P V; the half-tile's products are summed from zero
+//    before they reach the accumulator (added one MFMA at a time to an
+//    accumulator dominated by one large weight, small weights lose bits in the
+//    same direction at every step: 2.8e-5 on a row of one dominant key and
+//    4095 keys 2^-25 below it).
+//  * An infinity or NaN (or a value that rounds to one in BF16) has no parts.
+//    Such a half, and every half of a wavefront with such a query row, takes
+//    the FP32 MFMAs on values read from global memory (direct_scores,
+//    direct_values).
+// Measured against v_mfma_f32_16x16x4_f32 throughout, 64-bit errors beside:
+// 4 x 384..1024 tokens, 16/4 heads 132.3 -> 93.4 us (3.3e-7 -> 2.0e-7), 813
+// tokens, 12/1 heads 63.8 -> 45.6 (4.0e-7 -> 2.5e-7), 8 x 4096 tokens, 32/8
+// heads 8874 -> 6411 us (3.7e-7 -> 2.4e-7). What bounds it now is LDS reads
+// (384 KiB per half and workgroup, 128 bytes a clock: 1.3 of 2.8 us) beside
+// 96 MFMAs per wavefront and half (1.3 us).
+template <int kD>
+__global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillParams p) {
+    using M = PfBf16Exact;
+    using Vec = M::Vec;
+    constexpr int kKeys = 32;                  // keys per step
+    constexpr int kSteps = kD / 32, kDt = kD / 16, kCpr = kD / 8;
+    constexpr int kRowBytes = kD * 2;          // a key row of one part
+    constexpr int kPartBytes = kKeys * kRowBytes;
+    constexpr int kLoads = 2 * kKeys * kCpr / kPfThreads;  // 8-value chunks per thread and half, K's before V's
+    constexpr int kVSwz = kCpr / 8;
+    constexpr float kLazy = M::kLazyLog2;
+    static_assert(kLoads >= 1 && 2 * kKeys * kCpr % kPfThreads == 0, "half split");
+    // [buffer][K, V][part]
+    __shared__ __attribute__((aligned(16))) unsigned char parts_lds[2][2][3][kPartBytes];
+    __shared__ std::uint32_t pages[pf_table_max<kD>()];
+    __shared__ std::uint32_t no_parts[2];      // per buffer: 1 + the last half with a value without parts
+
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+    const int col = lane % 16, quad = lane / 16;
+    const std::uint32_t kvh = blockIdx.x % p.heads;
+    const PfShare share = pf_share<kD>(p);
+    if (share.idle) return;  // uniform
+    const std::uint32_t kv_len = share.kv_len, t0 = share.t0, past = share.past, last_key = share.last_key;
+    const std::uint64_t* const table = share.table;
+    // Pages of every key of the last half, whose keys past last_key are loaded too.
+    const std::uint32_t npages = ((last_key | (kKeys - 1)) >> p.bs_shift) + 1;
+    constexpr std::uint32_t kWin = pf_table_max<kD>();
+    // Halves per page window - 1 (windows start at multiples of kWin pages; a
+    // window holds at least 2048 keys).
+    const std::uint32_t win_mask = static_cast<std::uint32_t>((static_cast<std::uint64_t>(kWin) << p.bs_shift) / kKeys) - 1;
+    auto stage = [&](std::uint32_t first) {
+        for (std::uint32_t i = tid; i < kWin && first + i < npages; i += kPfThreads) {
+            const std::uint32_t pg = first + i;
+            const std::uint64_t id = pg < share.table_len ? table[pg] : p.num_blocks;
+            pages[i] = id < p.num_blocks ? static_cast<std::uint32_t>(id) : kPfMissing;
+        }
+    };
+    const std::uint32_t half_begin = 2 * share.tile_begin;
+    std::uint32_t half_end = 2 * share.tile_end;
+    if (half_end > last_key / kKeys + 1) half_end = last_key / kKeys + 1;
+
+    // This lane's query row, 32-bit values: scaled, in three parts.
+    const std::uint32_t r = static_cast<std::uint32_t>(16 * wave + col);
+    const std::uint32_t head = r % p.q_pass, token = t0 + r / p.q_pass;
+    const std::uint64_t q_row =
+        static_cast<std::uint64_t>(token < share.tq ? token : share.tq - 1) * p.query_heads + kvh * p.q_group + p.q_first + head;
+    const float* const q_src = share.query + q_row * kD + 8 * quad;
+    float4 qraw[kSteps][2];
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) qraw[kk][i] = *reinterpret_cast<const float4*>(q_src + 32 * kk + 4 * i);
+    stage((half_begin & ~win_mask) * kKeys >> p.bs_shift);
+    if (tid < 2) no_parts[tid] = 0;
+
+    // Eight values to 16 bytes of each part; false when some value has none
+    // (the last remainder is then not a number).
+    auto split8 = [](const float4& a, const float4& b, uint4 (&out)[3]) -> bool {
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        std::uint32_t w[3][4];
+        float rest = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pf_f32x2_t v{x[2 * j], x[2 * j + 1]};
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const pf_bf16x2_t h = __builtin_convertvector(v, pf_bf16x2_t);
+                w[i][j] = __builtin_bit_cast(std::uint32_t, h);
+                v -= __builtin_convertvector(h, pf_f32x2_t);
+            }
+            rest = max3(rest, v[0], v[1]);  // propagates NaN
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) out[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+        return rest == rest;
+    };
+    Vec qop[3][kSteps];
+    bool q_parts = true;
+#pragma unroll
+    for (int kk = 0; kk < kSteps; ++kk) {
+        const float4 lo = qraw[kk][0], hi = qraw[kk][1];
+        const float sc = p.scale_log2;
+        uint4 w[3];
+        q_parts &= split8(make_float4(lo.x * sc, lo.y * sc, lo.z * sc, lo.w * sc),
+                          make_float4(hi.x * sc, hi.y * sc, hi.z * sc, hi.w * sc), w);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) qop[i][kk] = __builtin_bit_cast(Vec, w[i]);
+    }
+    const bool wave_direct = __builtin_amdgcn_ballot_w64(!q_parts) != 0;
+    __syncthreads();  // pages[] and no_parts[] ready
+
+    const float* const kc = static_cast<const float*>(p.key_cache);
+    const float* const vc = static_cast<const float*>(p.value_cache);
+    const std::uint64_t page_elems = (static_cast<std::uint64_t>(kD) << p.bs_shift) * p.heads;
+    const std::uint32_t in_page_mask = (1u << p.bs_shift) - 1;
+    auto kswz = [](int row) { return kCpr >= 16 ? (row & 15) : ((row >> 1) & 7); };
+    auto vswz = [](int row) { return kVSwz * (row & 7); };
+    // Element offset of key `key`'s row in page `page`.
+    auto row_at = [&](std::uint32_t page, std::uint32_t key) {
+        return page * page_elems + (static_cast<std::uint64_t>((kvh << p.bs_shift) + (key & in_page_mask))) * kD;
+    };
+
+    // Chunk e of a half: values 8 * (e % kCpr) .. of key (e / kCpr) % 32, of K
+    // for e < 32 * kCpr and of V after. Keys past the sequence and missing
+    // pages read as zeros (the pool's first row is loaded instead, so every
+    // load is unconditional).
+    struct Chunk { float4 lo, hi; };
+    Chunk held[kLoads];
+    bool live[kLoads];
+    auto fetch = [&](std::uint32_t half) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int e = i * kPfThreads + tid;
+            const int row = (e / kCpr) % kKeys, c = e % kCpr;
+            const std::uint32_t key = half * kKeys + row;
+            const std::uint32_t slot = ((half & win_mask) * kKeys + row) >> p.bs_shift;
+            const std::uint32_t entry = key < kv_len ? pages[slot] : kPfMissing;
+            live[i] = !(entry & kPfMissing);
+            const float* src = (e < kKeys * kCpr ? kc : vc) + (live[i] ? row_at(entry, key) : 0) + 8 * c;
+            held[i].lo = *reinterpret_cast<const float4*>(src);
+            held[i].hi = *reinterpret_cast<const float4*>(src + 4);
+        }
+    };
+    auto convert = [&](std::uint32_t half) {
+        const int buf = half & 1;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int e = i * kPfThreads + tid;
+            const int kv = e < kKeys * kCpr ? 0 : 1, row = (e / kCpr) % kKeys, c = e % kCpr;
+            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            uint4 w[3];
+            const bool ok = split8(live[i] ? held[i].lo : zero, live[i] ? held[i].hi : zero, w);
+            const int at = row * kRowBytes + (c ^ (kv == 0 ? kswz(row) : vswz(row))) * 16;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(&parts_lds[buf][kv][k][at]) = w[k];
+            if (!ok) no_parts[buf] = half + 1;  // every writer of a half stores the same
+        }
+    };
+
+    std::uint32_t v_read0;
+    {
+        const int s = lane % 16, row = 4 * quad + s / 4;
+        const int c = (4 * (s % 4)) / 8;
+        v_read0 = row * kRowBytes + ((c ^ vswz(row)) * 16) + (s % 2) * 8;
+    }
+    const std::uint32_t k_read0 = col * kRowBytes + (quad ^ kswz(col)) * 16;
+
+    pf_f32x4_t acc[kDt];
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) acc[dt] = pf_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    pf_f32x4_t nref{0.0f, 0.0f, 0.0f, 0.0f};  // minus the reference point, in every lane of the vector
+    float sum_hi = 0.0f, sum_lo = 0.0f;       // this lane's weights of the row (compensated)
+    bool have_ref = false;
+    const pf_f32x4_t zero4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // A half without parts: v_mfma_f32_16x16x4_f32 on values read from global
+    // memory. Key row of the half; zeros past the sequence and in missing pages.
+    auto direct_row = [&](const float* cache, std::uint32_t key) -> const float* {
+        const std::uint32_t pg = key >> p.bs_shift;
+        if (key >= kv_len || pg >= share.table_len || table[pg] >= p.num_blocks)
+            return reinterpret_cast<const float*>(pf_zero_rows);
+        return cache + row_at(static_cast<std::uint32_t>(table[pg]), key);
+    };
+    auto direct_scores = [&](std::uint32_t half, pf_f32x4_t (&s)[2]) {
+#pragma unroll 1
+        for (int kt2 = 0; kt2 < 2; ++kt2) {
+            const float* row = direct_row(kc, half * kKeys + 16 * kt2 + col) + 8 * quad;
+            pf_f32x4_t t = nref;
+#pragma unroll 1
+            for (int i = 0; i < 8 * kSteps; ++i) {  // dim 32 * (i / 8) + 8 * quad + i % 8
+                const int d = 32 * (i / 8) + i % 8;
+                t = __builtin_amdgcn_mfma_f32_16x16x4f32(row[d], q_src[d] * p.scale_log2, t, 0, 0, 0);
+            }
+            s[kt2] = t;
+        }
+    };
+    auto direct_values = [&](std::uint32_t half, const float (&pr)[8]) {
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) {
+            pf_f32x4_t t = zero4;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float* row = direct_row(vc, half * kKeys + 16 * (i / 4) + 4 * quad + i % 4);
+                t = __builtin_amdgcn_mfma_f32_16x16x4f32(row[16 * dt + col], pr[i], t, 0, 0, 0);
+            }
+            acc[dt] += t;
+        }
+    };
+
+    const std::uint32_t min_limit = past + t0;
+    auto compute = [&](std::uint32_t half) {
+        const int buf = half & 1;
+        const std::uint32_t k0 = half * kKeys;
+        const bool direct =
+            wave_direct || static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(no_parts[buf])) == half + 1;
+        pf_f32x4_t s[2];
+        if (__builtin_expect(direct, 0)) {
+            direct_scores(half, s);
+        } else {
+            // Large products (hi hi, hi mid, mid hi) and small ones apart: four
+            // chains of 3 * kSteps MFMAs.
+            pf_f32x4_t small[2] = {zero4, zero4};
+            s[0] = nref;
+            s[1] = nref;
+#pragma unroll
+            for (int kk = 0; kk < kSteps; ++kk)
+#pragma unroll
+                for (int kt2 = 0; kt2 < 2; ++kt2) {
+                    Vec a[3];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        a[k] = __builtin_bit_cast(
+                            Vec, *reinterpret_cast<const uint4*>(&parts_lds[buf][0][k][16 * kt2 * kRowBytes + (k_read0 ^ (kk << 6))]));
+                    small[kt2] = M::mma(a[2], qop[0][kk], small[kt2]);
+                    s[kt2] = M::mma(a[1], qop[0][kk], s[kt2]);
+                    small[kt2] = M::mma(a[1], qop[1][kk], small[kt2]);
+                    s[kt2] = M::mma(a[0], qop[1][kk], s[kt2]);
+                    small[kt2] = M::mma(a[0], qop[2][kk], small[kt2]);
+                    s[kt2] = M::mma(a[0], qop[0][kk], s[kt2]);
+                }
+            s[0] += small[0];
+            s[1] += small[1];
+        }
+        if (k0 + kKeys - 1 > min_limit) {
+            const std::int32_t room = static_cast<std::int32_t>(past + token - k0 - 4 * quad);
+#pragma unroll
+            for (int kt2 = 0; kt2 < 2; ++kt2)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[kt2][i] = 16 * kt2 + i > room ? -INFINITY : s[kt2][i];
+        }
+        const float lmax = max3(max3(s[0][0], s[0][1], s[0][2]), max3(s[0][3], s[1][0], s[1][1]),
+                                max3(s[1][2], s[1][3], -INFINITY));
+        const bool grow = !have_ref || lmax > kLazy;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(grow) != 0, 0)) {
+            const float tmax = max_across_quads(lmax);
+            const float shift = !have_ref || tmax > kLazy ? tmax : 0.0f;
+            const float alpha = __builtin_amdgcn_exp2f(fminf(-shift, 0.0f));
+            nref -= shift;
+            sum_hi *= alpha;
+            sum_lo *= alpha;
+            s[0] -= shift;
+            s[1] -= shift;
+#pragma unroll
+            for (int dt = 0; dt < kDt; ++dt) acc[dt] *= alpha;
+            have_ref = true;
+        }
+        float pr[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pr[i] = __builtin_amdgcn_exp2f(s[i / 4][i % 4]);
+        two_sum_add(sum_hi, sum_lo, ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7])));
+        if (__builtin_expect(direct, 0)) {
+            direct_values(half, pr);
+            return;
+        }
+        Vec pb[3];
+        {
+            std::uint32_t w[3][4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                std::uint32_t x[3];
+                M::split3(pr[2 * j], pr[2 * j + 1], x);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) w[k][j] = x[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) pb[k] = __builtin_bit_cast(Vec, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
+        }
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) {
+            Vec a[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const auto* base = (__attribute__((address_space(3))) char*)(&parts_lds[buf][1][k][0]) + (v_read0 ^ (dt << 5));
+                const pf_i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4_t*)base);
+                const pf_i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pf_lds_i16x4_t*)(base + 16 * kRowBytes));
+                a[k] = __builtin_bit_cast(Vec, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+            pf_f32x4_t small = M::mma(a[2], pb[0], zero4), large = M::mma(a[1], pb[0], zero4);
+            small = M::mma(a[1], pb[1], small);
+            large = M::mma(a[0], pb[1], large);
+            small = M::mma(a[0], pb[2], small);
+            large = M::mma(a[0], pb[0], large);
+            acc[dt] += large + small;
+        }
+    };
+
+    // Half t lives in buffer t % 2. While t is computed, t + 1 goes from
+    // registers to its buffer (last read for t - 1, before the barrier) and the
+    // loads of t + 2 are in flight. fetch() of a page window's first half
+    // restages the page list: every wave is past its reads of the old one after
+    // the step's barrier.
+    auto fetch_next = [&](std::uint32_t half) {
+        if (half >= half_end) return;  // uniform
+        if ((half & win_mask) == 0 && half != half_begin) {
+            wait_lgkm0();
+            lds_barrier();
+            stage(half * kKeys >> p.bs_shift);
+            wait_lgkm0();
+            lds_barrier();
+        }
+        fetch(half);
+    };
+    if (half_begin < half_end) {  // uniform
+        fetch(half_begin);
+        convert(half_begin);
+        fetch_next(half_begin + 1);
+        wait_lgkm0();
+        lds_barrier();
+        for (std::uint32_t half = half_begin; half < half_end; ++half) {
+            if (half + 1 < half_end) {
+                convert(half + 1);
+                fetch_next(half + 2);
+            }
+            compute(half);
+            wait_lgkm0();
+            lds_barrier();
+        }
+    }
+
+    const float l = sum_across_quads(sum_hi + sum_lo);
+    if (token < share.t_end) {
+        // Normalised rows of the output, or unnormalised partials (an empty
+        // split leaves l = 0).
+        const bool whole = p.splits == 1;
+        const std::uint64_t prow = static_cast<std::uint64_t>(share.split) * share.tq * p.query_heads + q_row;
+        float* dst = whole ? share.output + q_row * kD : p.part_o + prow * kD;
+        const float sc = whole ? (l > 0.0f ? 1.0f / l : 0.0f) : 1.0f;
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt)
+            *reinterpret_cast<float4*>(dst + 16 * dt + 4 * quad) =
+                make_float4(acc[dt][0] * sc, acc[dt][1] * sc, acc[dt][2] * sc, acc[dt][3] * sc);
+        if (!whole && quad == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(-nref[0], l);
     }
 }
 
@@ -912,7 +1184,11 @@ int launch_prefill_pass(const PrefillParams& p, hipStream_t s) {
     const std::uint64_t grid = static_cast<std::uint64_t>(q.qblocks) * p.heads * (p.num_seqs ? p.num_seqs : p.splits);
     if (grid > 0xffffffffULL) return fail(KVFLUX_ERR_UNSUPPORTED, "paged prefill: %llu workgroups",
                                           static_cast<unsigned long long>(grid));
-    hipLaunchKernelGGL((paged_prefill_kernel<E, kD, kKs>), dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0, s, q);
+    if constexpr (std::is_same<E, PfF32>::value) {
+        hipLaunchKernelGGL((paged_prefill_f32_kernel<kD>), dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0, s, q);
+    } else {
+        hipLaunchKernelGGL((paged_prefill_kernel<E, kD, kKs>), dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0, s, q);
+    }
     return launch_status("paged_prefill_kernel");
 }
 
@@ -937,7 +1213,12 @@ int launch_prefill_group(const PrefillParams& p, std::uint32_t group, int key_pa
     for (std::uint32_t first = 0; first < group; first += sub) {
         q.q_first = first;
         // Key parts are chosen only for groups that fit half the rows.
-        const int st = key_parts == 2 ? launch_prefill_pass<E, kD, 2>(q, s) : launch_prefill_pass<E, kD, 1>(q, s);
+        int st;
+        if constexpr (std::is_same<E, PfF32>::value) {
+            st = launch_prefill_pass<E, kD, 1>(q, s);
+        } else {
+            st = key_parts == 2 ? launch_prefill_pass<E, kD, 2>(q, s) : launch_prefill_pass<E, kD, 1>(q, s);
+        }
         if (st != KVFLUX_OK) return st;
     }
     if (p.splits > 1) {
@@ -1003,11 +1284,11 @@ inline PrefillPlan prefill_most_splits(std::uint64_t head_size, std::uint64_t gr
 // kStep for loads and barriers; a launch takes the longest of its longest
 // workgroup and its work over all CUs, in whole rounds when the workgroups are
 // about equal (a query block behind a long prefix); splits add the partials'
-// way through memory, and two key parts have to promise a margin (more in
-// FP32, whose two 64-row workgroups load as much as one of 128).
+// way through memory, and two key parts (not in the FP32 kernel) have to
+// promise a margin, more in the exact variant's 64-row workgroups.
 // Measured, BF16, 32/8 heads, D = 128, one and two key parts: 16 workgroups of
 // the latter over 1024 keys 35.4 and 25.3 us, 256 of them 40 and 32; 512 (256
-// with one) 45.8 and 73. FP32: 138 and 75, 168 and 92, 168 and 187 us. One
+// with one) 45.8 and 73. One
 // prompt of 1500 tokens, exact: no split 75.8 us (119.3 with two splits and
 // their 49 MB of partials, about 8 more with two key parts); 512 tokens behind
 // 32768: 4 splits 247 us, 8 splits 275. `share`: the part of the largest
@@ -1016,15 +1297,15 @@ inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32,
                                   std::uint64_t num_kv_heads, std::uint64_t num_seqs, std::uint64_t kv_len,
                                   std::uint64_t query_tokens, std::uint64_t query_heads, std::uint64_t most_splits) {
     constexpr double kCus = 256, kStart = 10.0, kStep = 0.35, kBytesPerUs = 5e6;
-    // us of a tile's MFMAs in a workgroup (8 x 4096 tokens, and 4 x 1024 in FP32)
-    const double mfma = (f32 ? 8.7 : exact ? 2.5 : 1.7) * (f32 || exact ? head_size / 128.0 : 1.0);
+    // us of a tile's MFMAs in a workgroup, from 8 x 4096 tokens
+    const double mfma = (f32 ? 5.0 : exact ? 2.5 : 1.7) * (f32 || exact ? head_size / 128.0 : 1.0);
     const double share = num_seqs > 1 ? 0.6 : 1.0;
     const double margin = exact ? 1.25 : 1.05;
     const std::uint64_t tiles = (kv_len + kPfTile - 1) / kPfTile;
     const double past = static_cast<double>((kv_len - query_tokens) / kPfTile);
     PrefillPlan best{1, static_cast<std::uint32_t>(tiles), 0, 1};
     double best_time = 0;
-    for (int parts = 1; parts <= 2; ++parts) {
+    for (int parts = 1; parts <= (f32 ? 1 : 2); ++parts) {
         const std::uint64_t rows = 16 * (kPfWaves / parts) * pf_blocks_for(static_cast<int>(head_size), exact);
         if (parts == 2 && group > rows) break;
         const std::uint64_t sub = prefill_sub_group(static_cast<std::uint32_t>(group), static_cast<std::uint32_t>(rows));

@@ -108,3 +108,51 @@ def test_exact_key_parts(gpu, case):
         got = out.download(np.float32)
         assert np.all(got[q.size:] == 7.0) and np.all(np.isnan(ws.download(np.float32)[size // 4:]))
         assert np.abs(got[:q.size] - exp).max() < 1e-5
+
+
+@pytest.mark.parametrize("D,bs,kv,tq", [(128, 16, 200, 200), (64, 1, 2500, 40), (128, 4, 9000, 33)])
+def test_f32_values_without_parts(gpu, D, bs, kv, tq):
+    """FP32 caches enter BF16 MFMAs as three parts each; infinities and values
+    that round to one in BF16 have none. A key with an infinite element that
+    every row scores -inf drops out, V keeps values near the largest float,
+    and an infinite query element (first row) leaves the other rows alone."""
+    kv_heads, q_heads = 2, 8
+    code, host = DTYPES["Float32"]
+    kc, vc, blocks, table, width = arena("Float32", kv_heads, bs, D, [kv], 900 + kv)
+    kh, vh = kc.download(host).reshape(blocks, kv_heads, bs, D), vc.download(host).reshape(blocks, kv_heads, bs, D)
+    q = oracle.random_elements(0, tq * q_heads * D, oracle.F32, 1, 950).reshape(tq, q_heads, D)
+    q[:, :, 3] = -np.abs(q[:, :, 3]) - 3
+    at = lambda t: (int(table[0, t // bs]), slice(None), t % bs)  # noqa: E731
+    seen = kv - tq  # every row sees the keys up to here
+    # Not key 0: with tq == kv it is the first row's only key, and a row whose
+    # every score is -inf has no softmax.
+    dropped, big = seen // 2 + 1, max(seen - 40, 2)
+    kh[at(dropped)][:, 3] = np.inf
+    # Weights are relative to a reference point up to 2^8 below the largest
+    # score, so a key of ordinary score would overflow the sum itself: this one
+    # scores 3 * 30 / sqrt(D) (8 or more) below the others.
+    kh[at(big)][:, 3] = 30.0
+    vh[at(big)][:, 5] = 3.4e38
+    kc.upload(kh.reshape(-1))
+    vc.upload(vh.reshape(-1))
+    exp = oracle.paged_attention_causal(kh.reshape(-1), vh.reshape(-1), kv_heads, bs, D, code, table[0], kv,
+                                        q.reshape(-1), tq, q_heads, threads=8).reshape(tq, q_heads, D)
+    td = buffer_like(table.reshape(-1))
+    for bad_row in (False, True):
+        if bad_row:
+            q[0, 0, 7] = np.inf
+        qd, out = buffer_like(q.reshape(-1)), buffer_like(np.full(q.size, 7.0, np.float32))
+        capi.check(capi.lib().kvflux_paged_prefill(kc.ptr, vc.ptr, blocks, kv_heads, bs, D, code, td.ptr, width, kv,
+                                                   tq, q_heads, qd.ptr, out.ptr, None))
+        device.synchronize()
+        got = out.download(np.float32).reshape(tq, q_heads, D)
+        rest = np.ones((tq, q_heads), bool)
+        rest[0, 0] = not bad_row
+        # Rows that see the key dropped or the large value: relative there.
+        assert np.all(np.isfinite(got[rest]))
+        err = np.abs(got.astype(np.float64) - exp) / np.maximum(1.0, np.abs(exp))
+        # Column 5 is the large value times one weight, whose relative error
+        # is ln 2 times its score's: scores down to -64 (log2) round at 2^-19
+        # in each of the kernel's up to 32 steps, 32 * 2^-19 * ln 2 = 4.3e-5.
+        assert np.delete(err, 5, axis=2)[rest].max() < 1e-5
+        assert err[rest][:, 5].max() < 5e-5
