@@ -48,6 +48,7 @@ namespace {
 constexpr int kThreads = 512;
 constexpr int kLiveVpt = 2;   // vectors per thread, live-page launch
 constexpr int kTableVpt = 2;  // vectors per thread, table launch
+constexpr std::uint32_t kSmallPage = kThreads * kLiveVpt / 2;  // vectors of a page moved by wavefronts
 
 // Shape of one page and of one output token, in vectors.
 struct PageShape {
@@ -59,18 +60,19 @@ struct PageShape {
 
 // Part `part` of a page whose first `valid` tokens are live: src is the
 // page's first vector in the cache, dst the page's first output vector.
-template <typename Vec, int kVpt>
+// `lane` of the kGroup threads that move it.
+template <typename Vec, int kVpt, int kGroup>
 __device__ inline void gather_part(const Vec* __restrict__ src, Vec* __restrict__ dst, std::uint32_t valid,
-                                   std::uint32_t part, const PageShape& shape) {
+                                   std::uint32_t part, std::uint32_t lane, const PageShape& shape) {
     const std::uint32_t live_vectors = valid * shape.token_vectors.divisor;
-    const std::uint32_t first = part * (kThreads * kVpt);
+    const std::uint32_t first = part * (kGroup * kVpt);
     if (first >= live_vectors) return;  // uniform: the part lies past the tail
     const std::uint32_t vpr = shape.row_vectors.divisor;
     Vec r[kVpt];
     bool live[kVpt];
 #pragma unroll
     for (int u = 0; u < kVpt; ++u) {
-        const std::uint32_t j = first + u * kThreads + threadIdx.x;  // output order
+        const std::uint32_t j = first + u * kGroup + lane;  // output order
         live[u] = j < live_vectors;
         const std::uint32_t token = shape.token_vectors.div(j);
         const std::uint32_t rest = j - token * shape.token_vectors.divisor;
@@ -83,7 +85,7 @@ __device__ inline void gather_part(const Vec* __restrict__ src, Vec* __restrict_
     for (int u = 0; u < kVpt; ++u) keep_in_registers(r[u]);
 #pragma unroll
     for (int u = 0; u < kVpt; ++u) {
-        if (live[u]) stream_store(dst + first + u * kThreads + threadIdx.x, r[u]);
+        if (live[u]) stream_store(dst + first + u * kGroup + lane, r[u]);
     }
 }
 
@@ -109,15 +111,20 @@ __device__ inline std::uint32_t find_sequence(const std::uint64_t* __restrict__ 
     return lo;
 }
 
-template <typename Vec>
+// kGroup threads (a workgroup, or a wavefront of it) move one part.
+template <typename Vec, int kVpt, int kGroup>
 __global__ __launch_bounds__(kThreads) void paged_kv_gather_live_kernel(
     const Vec* __restrict__ key_cache, const Vec* __restrict__ value_cache, std::uint64_t num_blocks,
     const std::uint64_t* __restrict__ block_table, std::uint64_t table_width,
     const std::uint64_t* __restrict__ seq_lens, const std::uint64_t* __restrict__ out_offsets,
     const std::uint64_t* __restrict__ page_starts, std::uint32_t num_seqs, Vec* __restrict__ key_out,
-    Vec* __restrict__ value_out, FastDiv parts, PageShape shape) {
-    const std::uint32_t w = parts.div(blockIdx.x);
-    const std::uint32_t part = blockIdx.x - w * parts.divisor;
+    Vec* __restrict__ value_out, FastDiv parts, std::uint32_t units, PageShape shape) {
+    constexpr std::uint32_t kGroups = kThreads / kGroup;
+    const std::uint32_t group = kGroups == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x / kGroup);
+    const std::uint32_t unit = blockIdx.x * kGroups + group;
+    if (unit >= units) return;  // uniform in the group
+    const std::uint32_t w = parts.div(unit);
+    const std::uint32_t part = unit - w * parts.divisor;
     const std::uint32_t seq = __builtin_amdgcn_readfirstlane(find_sequence(page_starts, num_seqs, w));
     const std::uint64_t first_page = page_starts[seq];
     if (w < first_page) return;  // malformed scan
@@ -132,7 +139,7 @@ __global__ __launch_bounds__(kThreads) void paged_kv_gather_live_kernel(
     const std::uint32_t valid = remaining < shape.block_size ? static_cast<std::uint32_t>(remaining) : shape.block_size;
     const Vec* src = (blockIdx.z == 0 ? key_cache : value_cache) + page * shape.page_vectors;
     Vec* dst = (blockIdx.z == 0 ? key_out : value_out) + (out_first + first_token) * shape.token_vectors.divisor;
-    gather_part<Vec, kLiveVpt>(src, dst, valid, part, shape);
+    gather_part<Vec, kVpt, kGroup>(src, dst, valid, part, threadIdx.x % kGroup, shape);
 }
 
 template <typename Vec>
@@ -155,7 +162,7 @@ __global__ __launch_bounds__(kThreads) void paged_kv_gather_kernel(
     const std::uint32_t valid = remaining < shape.block_size ? static_cast<std::uint32_t>(remaining) : shape.block_size;
     const Vec* src = (blockIdx.z == 0 ? key_cache : value_cache) + page * shape.page_vectors;
     Vec* dst = (blockIdx.z == 0 ? key_out : value_out) + (out_first + first_token) * shape.token_vectors.divisor;
-    gather_part<Vec, kTableVpt>(src, dst, valid, part, shape);
+    gather_part<Vec, kTableVpt, kThreads>(src, dst, valid, part, threadIdx.x, shape);
 }
 
 // Validation shared by both entries; fills `shape` and the vector width.
@@ -218,19 +225,43 @@ int launch_table(const void* kc, const void* vc, std::uint64_t num_blocks, const
     return KVFLUX_OK;
 }
 
+template <typename Vec, int kVpt, int kGroup>
+int launch_live_parts(const void* kc, const void* vc, std::uint64_t num_blocks, const PageShape& shape,
+                      const std::uint64_t* table, std::uint64_t width, const std::uint64_t* lens,
+                      const std::uint64_t* offsets, const std::uint64_t* starts, std::uint64_t num_seqs,
+                      std::uint64_t total_pages, void* ko, void* vo, hipStream_t s) {
+    constexpr std::uint64_t kPart = static_cast<std::uint64_t>(kGroup) * kVpt, kGroups = kThreads / kGroup;
+    const std::uint64_t parts = (shape.page_vectors + kPart - 1) / kPart;
+    if (total_pages * parts > 0x7fffffffULL) return fail(KVFLUX_ERR_UNSUPPORTED, "gather: too many pages");
+    const auto units = static_cast<std::uint32_t>(total_pages * parts);
+    const dim3 grid(static_cast<unsigned>((units + kGroups - 1) / kGroups), 1, 2);
+    hipLaunchKernelGGL((paged_kv_gather_live_kernel<Vec, kVpt, kGroup>), grid, dim3(kThreads), 0, s,
+                       static_cast<const Vec*>(kc), static_cast<const Vec*>(vc), num_blocks, table, width, lens,
+                       offsets, starts, static_cast<std::uint32_t>(num_seqs), static_cast<Vec*>(ko),
+                       static_cast<Vec*>(vo), FastDiv(static_cast<std::uint32_t>(parts)), units, shape);
+    return launch_status("paged_kv_gather_live_kernel");
+}
+
+// Pages of at most half a workgroup's part leave most of its threads without
+// a vector: there every wavefront takes parts of its own, of two vectors a
+// lane (one where a page has no more than 64). 32 sequences of U[512, 4096]
+// tokens, pages of 64, 128, 256 and 512 vectors, a workgroup and a wavefront
+// per part: 36.0 and 9.0 us, 41.8 and 15.0, 49.5 and 27.2, 59.2 and 52.7
+// (1.1 -> 4.5 TB/s up to 5.45 -> 6.1); from 1024 vectors on both fill their
+// threads and the workgroup searches once for eight wavefronts' worth.
 template <typename Vec>
 int launch_live(const void* kc, const void* vc, std::uint64_t num_blocks, const PageShape& shape,
                 const std::uint64_t* table, std::uint64_t width, const std::uint64_t* lens,
                 const std::uint64_t* offsets, const std::uint64_t* starts, std::uint64_t num_seqs,
                 std::uint64_t total_pages, void* ko, void* vo, hipStream_t s) {
-    const std::uint64_t parts = (shape.page_vectors + kThreads * kLiveVpt - 1) / (kThreads * kLiveVpt);
-    if (total_pages * parts > 0x7fffffffULL) return fail(KVFLUX_ERR_UNSUPPORTED, "gather: too many pages");
-    const dim3 grid(static_cast<unsigned>(total_pages * parts), 1, 2);
-    hipLaunchKernelGGL(paged_kv_gather_live_kernel<Vec>, grid, dim3(kThreads), 0, s, static_cast<const Vec*>(kc),
-                       static_cast<const Vec*>(vc), num_blocks, table, width, lens, offsets, starts,
-                       static_cast<std::uint32_t>(num_seqs), static_cast<Vec*>(ko), static_cast<Vec*>(vo),
-                       FastDiv(static_cast<std::uint32_t>(parts)), shape);
-    return launch_status("paged_kv_gather_live_kernel");
+    if (shape.page_vectors > kSmallPage || total_pages > 0x7fffffffULL / kSmallPage)
+        return launch_live_parts<Vec, kLiveVpt, kThreads>(kc, vc, num_blocks, shape, table, width, lens, offsets, starts,
+                                                          num_seqs, total_pages, ko, vo, s);
+    if (shape.page_vectors > 64)
+        return launch_live_parts<Vec, 2, 64>(kc, vc, num_blocks, shape, table, width, lens, offsets, starts, num_seqs,
+                                             total_pages, ko, vo, s);
+    return launch_live_parts<Vec, 1, 64>(kc, vc, num_blocks, shape, table, width, lens, offsets, starts, num_seqs,
+                                         total_pages, ko, vo, s);
 }
 
 } // namespace
