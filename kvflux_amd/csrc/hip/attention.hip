@@ -1844,12 +1844,18 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             }
             // Up to kAdaptRows rows the kernel, which knows the lengths,
             // takes the size from there on that balances the grid best.
-            std::uint32_t item = 1u << shift, item_max = item;
+            std::uint32_t item = 1u << shift, item_max;
             const std::uint64_t fine = fine_items(rows, p.kv_len, p.heads, p.query_heads, bs, kD);
             if (fine > 0 && scratch_bytes >= fine && kFineItem < item) item = kFineItem;
+            // Rows of one item at most need no partials: the item is as long
+            // as the longest may be, in whole steps (an item loads and masks
+            // all its tiles: 100 rows of 10-80 tokens in 512-token items
+            // 29.6 us, in 128-token items 14.8; one row of 30: 12.0 and 7.6).
+            const bool whole_rows = p.kv_len < item;
+            if (whole_rows) item = p.kv_len <= kItemStep ? kItemStep : static_cast<std::uint32_t>(p.kv_len + kItemStep - 1) / kItemStep * kItemStep;
             const std::uint64_t chunks = (p.kv_len + item - 1) / item;
             const std::uint64_t items = rows * chunks * p.heads * sets;  // upper bound of the real count
-            if (rows <= kAdaptRows && items <= 0x7fffffffULL) item_max = 1u << max_item_shift(bs);
+            item_max = !whole_rows && rows <= kAdaptRows && items <= 0x7fffffffULL ? 1u << max_item_shift(bs) : item;
             plan->family = Family::Bs16;
             plan->sub = sub;
             plan->small = small;

@@ -34,6 +34,8 @@ CASES = [
     # dtype, kv heads, q heads, D, block size, lengths
     ("BFloat16", 8, 32, 128, 16, [127, 128, 129, 1500]),
     ("BFloat16", 2, 8, 128, 16, [300]),
+    ("Float16", 2, 8, 128, 16, [1, 80, 128, 17, 0]),  # one item a row, no partials
+    ("BFloat16", 2, 14, 64, 4, [129, 200, 2]),
     ("Float16", 4, 28, 128, 16, [0, 1, 640, 641, 2047, 2048, 2049, 4000]),
     ("Float32", 2, 8, 128, 8, [1, 255, 257, 900]),
     ("BFloat16", 1, 4, 64, 1, [1, 256, 257, 400]),
