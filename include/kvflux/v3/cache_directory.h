@@ -20,6 +20,8 @@
 
 namespace kvflux::v3 {
 
+class GpuCpuTransfer;
+
 enum class ChunkState { READY, COPYING, LOADING, EVICTING, ERROR };
 
 // Identity of a KV chunk, independent of where it is stored: model, layout
@@ -116,6 +118,14 @@ private:
     // references); destroyed records leave a vacant entry for the next
     // create(). The index maps a key to its slab entry.
     ChunkRecord& record(const CacheKey& key);
+    ChunkRecord* find(const CacheKey& key) noexcept;  // null for an unknown key
+    // The calls above on a record already looked up: hashing a key costs as
+    // much as the rest of such a call, and a transfer makes several per chunk.
+    TierLocation place_in(ChunkRecord& rec, StorageTier tier, ChunkState state);
+    void remove_from(ChunkRecord& rec, StorageTier tier);
+    static void set_state_in(ChunkRecord& rec, StorageTier tier, ChunkState state);
+    static void unpin_in(ChunkRecord& rec);
+    friend class GpuCpuTransfer;
     // Position of `tier` in tiers_ / replicas_ (std::invalid_argument for a
     // value outside the enum).
     static std::size_t tier_index(StorageTier tier);

@@ -74,10 +74,11 @@ private:
     void begin(const std::vector<CacheKey>& keys, bool offload);
     // Takes the chunk's ticket once its copy has completed; std::logic_error
     // when no copy of the chunk is in flight or it lands in the other tier.
-    Ticket redeem(const CacheKey& key, StorageTier lands_in);
+    Ticket redeem(const ChunkRecord* record, StorageTier lands_in);
     // Moves the replicas out of their in-flight states (after checking they
     // are still the ones the ticket names) and drops the source on request.
-    void settle(const CacheKey& key, const Ticket& ticket, bool drop_source);
+    void settle(ChunkRecord& record, const Ticket& ticket, bool drop_source);
+    void finish(const CacheKey& key, StorageTier lands_in, bool drop_source);
     std::shared_ptr<Batch> acquire_batch(std::size_t pairs);
 
     CacheDirectory& directory_;
