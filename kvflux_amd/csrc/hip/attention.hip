@@ -1820,12 +1820,20 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             if (!small && kD != 256 && g > 8 && sub < 4) {
                 sub = g > 16 && g % 16 <= 8 ? 16u : 8u;
                 rest = g % sub;
+            } else if ((small || kD == 256) && g > cap && sub < 4) {
+                // The same for the shapes of at most `cap` heads an item: sets of
+                // that many and the rest (24 rows of U[500, 12000] tokens, 28/4
+                // heads, as seven sets of one head and as 5 + 2: 8-token pages
+                // at 128 197.8 and 99.5 us, head size 256 366 and 189).
+                sub = cap;
+                rest = g % sub;
             }
             const std::uint64_t sets = g / sub;  // head sets per kv head, each its own work items
             if (2 * rows * max_chunks * p.heads * sets > 0xffffffffULL) return plan_fallback(kD, group, max_chunks, plan);
             int rest_slots = 0;
             if (rest > 0) {
-                const int st = resident_slots_for<E, kD, false>(rest, &rest_slots);
+                const int st = small ? resident_slots_for<E, kD, true>(rest, &rest_slots)
+                                     : resident_slots_for<E, kD, false>(rest, &rest_slots);
                 if (st != KVFLUX_OK) return st;
             }
             int slots = 0;

@@ -41,6 +41,10 @@ CASES = [
     ("BFloat16", 1, 4, 64, 1, [1, 256, 257, 400]),
     ("Float16", 1, 11, 64, 64, [20000, 3]),  # a second launch for the heads past the sets
     ("BFloat16", 2, 10, 256, 32, [513, 5000]),
+    ("BFloat16", 2, 14, 128, 8, [700, 3]),      # small pages: sets of 5 heads and a launch for the other 2
+    ("Float16", 1, 7, 256, 16, [129, 2000]),    # head size 256 the same
+    ("Float16", 1, 13, 64, 4, [1000, 513]),     # small pages at 64: 8 and 5
+    ("Float32", 1, 11, 128, 8, [1000, 16]),
     ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(256)]),
     ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(257)]),
     ("Float32", 1, 1, 96, 16, [40000, 511, 512, 513]),  # the split kernel's partials, more than 64 of them
