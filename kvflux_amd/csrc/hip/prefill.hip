@@ -1291,26 +1291,26 @@ inline PrefillPlan prefill_most_splits(std::uint64_t head_size, std::uint64_t gr
 // with one) 45.8 and 73. One
 // prompt of 1500 tokens, exact: no split 75.8 us (119.3 with two splits and
 // their 49 MB of partials, about 8 more with two key parts); 512 tokens behind
-// 32768: 4 splits 247 us, 8 splits 275. `share`: the part of the largest
-// case's work to expect (ragged batches, whose lengths the host has not got).
+// 32768: 4 splits 247 us, 8 splits 275.
+// key_parts_allowed: not for kvflux_paged_prefill and the batch entry, whose
+// outputs are the same bits whatever else is in the launch.
 inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32, std::uint64_t group,
-                                  std::uint64_t num_kv_heads, std::uint64_t num_seqs, std::uint64_t kv_len,
-                                  std::uint64_t query_tokens, std::uint64_t query_heads, std::uint64_t most_splits) {
+                                  std::uint64_t num_kv_heads, std::uint64_t kv_len, std::uint64_t query_tokens,
+                                  std::uint64_t query_heads, std::uint64_t most_splits, bool key_parts_allowed) {
     constexpr double kCus = 256, kStart = 10.0, kStep = 0.35, kBytesPerUs = 5e6;
     // us of a tile's MFMAs in a workgroup, from 8 x 4096 tokens
     const double mfma = (f32 ? 5.0 : exact ? 2.5 : 1.7) * (f32 || exact ? head_size / 128.0 : 1.0);
-    const double share = num_seqs > 1 ? 0.6 : 1.0;
     const double margin = exact ? 1.25 : 1.05;
     const std::uint64_t tiles = (kv_len + kPfTile - 1) / kPfTile;
     const double past = static_cast<double>((kv_len - query_tokens) / kPfTile);
     PrefillPlan best{1, static_cast<std::uint32_t>(tiles), 0, 1};
     double best_time = 0;
-    for (int parts = 1; parts <= (f32 ? 1 : 2); ++parts) {
+    for (int parts = 1; parts <= (f32 || !key_parts_allowed ? 1 : 2); ++parts) {
         const std::uint64_t rows = 16 * (kPfWaves / parts) * pf_blocks_for(static_cast<int>(head_size), exact);
         if (parts == 2 && group > rows) break;
         const std::uint64_t sub = prefill_sub_group(static_cast<std::uint32_t>(group), static_cast<std::uint32_t>(rows));
         const std::uint64_t tok = rows / sub;
-        const double blocks = static_cast<double>((query_tokens + tok - 1) / tok * num_kv_heads) * num_seqs * (group / sub);
+        const double blocks = static_cast<double>((query_tokens + tok - 1) / tok * num_kv_heads) * (group / sub);
         const double mean_tiles = 0.5 * (past + static_cast<double>(tiles)) + 0.5;
         const double tile_time = mfma / parts + kStep;
         for (std::uint64_t want = 1; want <= most_splits; ++want) {
@@ -1323,7 +1323,7 @@ inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32,
             if (wgs <= kCus || past >= split_tiles) {
                 time = std::ceil(wgs / kCus) * longest;
             } else {
-                const double even = share * (blocks * mean_tiles * tile_time + wgs * kStart) / kCus;
+                const double even = (blocks * mean_tiles * tile_time + wgs * kStart) / kCus;
                 time = std::fmax(longest, even + 0.25 * longest);
             }
             const double partials = static_cast<double>(splits * query_tokens * query_heads * head_size) * 2 * sizeof(float);
@@ -1351,7 +1351,7 @@ int paged_prefill(const void* key_cache, const void* value_cache, uint64_t num_b
                   uint64_t block_size, uint64_t head_size, int dtype, const uint64_t* block_table,
                   uint64_t num_table_blocks, uint64_t kv_len, uint64_t query_tokens, uint64_t query_heads,
                   const float* query, float* output, void* workspace, uint64_t workspace_bytes, void* stream,
-                  bool exact = false) {
+                  bool key_parts_allowed, bool exact = false) {
     if (query_tokens == 0) return KVFLUX_OK;
     if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
     if (!key_cache || !value_cache || !block_table || !query || !output) {
@@ -1404,8 +1404,8 @@ int paged_prefill(const void* key_cache, const void* value_cache, uint64_t num_b
         }
         most_splits = most.splits;
     }
-    const PrefillPlan plan = prefill_choice(head_size, exact, dtype == KVFLUX_DTYPE_F32, group, num_kv_heads, 1, kv_len,
-                                            query_tokens, query_heads, most_splits);
+    const PrefillPlan plan = prefill_choice(head_size, exact, dtype == KVFLUX_DTYPE_F32, group, num_kv_heads, kv_len,
+                                            query_tokens, query_heads, most_splits, key_parts_allowed);
     if (plan.splits > 1) {
         p.splits = plan.splits;
         p.split_tiles = plan.split_tiles;
@@ -1431,7 +1431,7 @@ extern "C" int kvflux_paged_prefill(const void* key_cache, const void* value_cac
                                     uint64_t query_tokens, uint64_t query_heads, const float* query,
                                     float* output, void* stream) {
     return paged_prefill(key_cache, value_cache, num_blocks, num_kv_heads, block_size, head_size, dtype, block_table,
-                         num_table_blocks, kv_len, query_tokens, query_heads, query, output, nullptr, 0, stream);
+                         num_table_blocks, kv_len, query_tokens, query_heads, query, output, nullptr, 0, stream, false);
 }
 
 extern "C" int kvflux_paged_prefill_workspace_size(uint64_t num_kv_heads, uint64_t head_size, uint64_t kv_len,
@@ -1463,7 +1463,7 @@ extern "C" int kvflux_paged_prefill_split(const void* key_cache, const void* val
                                           float* output, void* workspace, uint64_t workspace_bytes, void* stream) {
     return paged_prefill(key_cache, value_cache, num_blocks, num_kv_heads, block_size, head_size, dtype, block_table,
                          num_table_blocks, kv_len, query_tokens, query_heads, query, output, workspace,
-                         workspace_bytes, stream);
+                         workspace_bytes, stream, true);
 }
 
 extern "C" int kvflux_paged_prefill_exact(const void* key_cache, const void* value_cache, uint64_t num_blocks,
@@ -1473,7 +1473,7 @@ extern "C" int kvflux_paged_prefill_exact(const void* key_cache, const void* val
                                           float* output, void* workspace, uint64_t workspace_bytes, void* stream) {
     return paged_prefill(key_cache, value_cache, num_blocks, num_kv_heads, block_size, head_size, dtype, block_table,
                          num_table_blocks, kv_len, query_tokens, query_heads, query, output, workspace,
-                         workspace_bytes, stream, true);
+                         workspace_bytes, stream, true, true);
 }
 
 extern "C" int kvflux_paged_prefill_batch(const void* key_cache, const void* value_cache, uint64_t num_blocks,
@@ -1529,10 +1529,7 @@ extern "C" int kvflux_paged_prefill_batch(const void* key_cache, const void* val
     p.seq_q_offsets = query_offsets;
     const hipStream_t s = as_stream(stream);
     const std::uint32_t g = static_cast<std::uint32_t>(query_heads / num_kv_heads);
-    const bool f32 = dtype == KVFLUX_DTYPE_F32;
-    const PrefillPlan plan = prefill_choice(head_size, f32, f32, g, num_kv_heads, num_seqs, max_kv_len,
-                                            max_query_tokens, query_heads, 1);
-    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, plan.key_parts, s);
-    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, plan.key_parts, s);
-    return launch_prefill_head_size<PfF16>(p, head_size, g, plan.key_parts, s);
+    if (dtype == KVFLUX_DTYPE_F32) return launch_prefill_head_size<PfF32>(p, head_size, g, 1, s);
+    if (dtype == KVFLUX_DTYPE_BF16) return launch_prefill_head_size<PfBf16>(p, head_size, g, 1, s);
+    return launch_prefill_head_size<PfF16>(p, head_size, g, 1, s);
 }

@@ -1,9 +1,8 @@
 """Prefill launches whose wavefronts split the keys of a workgroup (small
 grids): rows whose only keys lie in one half of a tile, last tiles with one or
 both halves live, groups at and past the halved row count, every dtype and
-head size, key splits beside them, and rows in different sequences of one
-batch. FP32 caches and the exact path at 1e-5 against the oracle over whole
-outputs, the rounded path at 2e-2.
+head size, and key splits beside them. FP32 caches and the exact path at 1e-5
+against the oracle over whole outputs, the rounded path at 2e-2.
 """
 from __future__ import annotations
 
@@ -37,7 +36,7 @@ def arena(name, kv_heads, bs, head_size, kv_lens, seed):
     return kc, vc, blocks, table, width
 
 
-BATCH = [  # name, kv heads, q heads, D, block size, (kv, queries) of each sequence
+SHAPES = [  # name, kv heads, q heads, D, block size, (kv, queries) of each sequence
     ("BFloat16", 2, 8, 128, 16, [(1, 1), (31, 31), (33, 33), (64, 64), (65, 65)]),
     ("Float16", 1, 4, 128, 8, [(97, 97), (320, 1), (352, 40), (130, 130)]),  # rows starting in either half
     ("BFloat16", 1, 128, 128, 16, [(70, 70)]),   # a group of exactly half the rows (one token a workgroup)
@@ -50,9 +49,9 @@ BATCH = [  # name, kv heads, q heads, D, block size, (kv, queries) of each seque
 ]
 
 
-@pytest.mark.parametrize("case", range(len(BATCH)))
-def test_batch_key_parts(gpu, case):
-    name, kv_heads, q_heads, D, bs, seqs = BATCH[case]
+@pytest.mark.parametrize("case", range(len(SHAPES)))
+def test_key_parts(gpu, case):
+    name, kv_heads, q_heads, D, bs, seqs = SHAPES[case]
     code, host = DTYPES[name]
     kv = np.array([a for a, _ in seqs], np.uint64)
     ql = np.array([b for _, b in seqs], np.uint64)
@@ -60,11 +59,13 @@ def test_batch_key_parts(gpu, case):
     kc, vc, blocks, table, width = arena(name, kv_heads, bs, D, kv, 700 + 2 * case)
     total, row = int(ql.sum()), q_heads * D
     q = oracle.random_elements(0, total * row, oracle.F32, 1, 750 + case)
-    td, qd, kd, ld, sd = (buffer_like(x) for x in (table.reshape(-1), q, kv, ql, off))
+    td, qd = buffer_like(table.reshape(-1)), buffer_like(q)
     out = buffer_like(np.full(total * row + 8, 7.0, np.float32))
-    capi.check(capi.lib().kvflux_paged_prefill_batch(kc.ptr, vc.ptr, blocks, kv_heads, bs, D, code, td.ptr, width,
-                                                     kd.ptr, ld.ptr, sd.ptr, len(seqs), int(ql.max()), int(kv.max()),
-                                                     q_heads, qd.ptr, out.ptr, None))
+    for i in range(len(seqs)):
+        at = int(off[i]) * row * 4
+        capi.check(capi.lib().kvflux_paged_prefill_split(kc.ptr, vc.ptr, blocks, kv_heads, bs, D, code,
+                                                         td.ptr + i * width * 8, width, int(kv[i]), int(ql[i]),
+                                                         q_heads, qd.ptr + at, out.ptr + at, None, 0, None))
     device.synchronize()
     got = out.download(np.float32)
     assert np.all(got[total * row:] == 7.0)
