@@ -911,7 +911,7 @@ def bench_prefill(v2, args, stream):
                                                       out_exact.ptr + i * T * Hq * D * 4, None, 0, stream))
 
     # FP32 caches holding the same values (BF16 widened exactly), one batch
-    # launch on FP32 MFMAs; the same oracle rows apply.
+    # launch; the same oracle rows apply.
     cache_bytes = storage.layout().cache_bytes()
     k32 = device.to_device((device.memcpy_d2h(kb, cache_bytes, np.uint16).astype(np.uint32) << 16).view(np.float32))
     v32 = device.to_device((device.memcpy_d2h(vb, cache_bytes, np.uint16).astype(np.uint32) << 16).view(np.float32))
@@ -977,7 +977,7 @@ def bench_prefill(v2, args, stream):
             "exact": {"ms": exact_ms, "TFLOPs": flops / (exact_ms * 1e-3) / 1e12,
                       "max_abs_err_vs_oracle": err_exact, "tolerance": 1e-5},
             # FP32 caches (the same values): one batch launch on
-            # v_mfma_f32_16x16x4_f32, against the FP32 MFMA peak.
+            # the three-part BF16 kernel, beside the FP32 MFMA peak.
             "f32": {"kernel": "paged_prefill_kernel<f32,128> (group 4), one batch launch", "ms": f32_ms,
                     "TFLOPs": flops / (f32_ms * 1e-3) / 1e12,
                     "frac_of_fp32_mfma_peak": flops / (f32_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS,

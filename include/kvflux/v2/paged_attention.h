@@ -17,7 +17,7 @@ namespace kvflux::v2 {
 //          uses it. Calls of 16 or more query tokens at head_size 64 or 128
 //          (block_size a power of two up to 256) run on the MFMA prefill:
 //          on a 16-bit cache with Q and the weights split into three 16-bit
-//          parts (exact products), on an FP32 cache with FP32 MFMAs; others
+//          parts (exact products), on an FP32 cache K and V as well; others
 //          on the split-K kernel.
 //   Auto:  Exact, except that calls of query_tokens >= 16 on a 16-bit cache
 //          at the shapes the MFMA prefill takes (head_size 64, 128 or 256,
@@ -25,7 +25,7 @@ namespace kvflux::v2 {
 //          softmax weights rounded to the cache dtype (2e-2 contract). FP32
 //          caches keep the Exact routing.
 //   Fast:  the MFMA prefill whenever the shape allows it (any query_tokens;
-//          rounded on 16-bit caches, FP32 MFMAs on FP32 caches), otherwise
+//          rounded on 16-bit caches, as Exact on FP32 caches), otherwise
 //          Exact.
 enum class AttentionPrecision { Exact, Auto, Fast };
 

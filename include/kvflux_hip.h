@@ -211,8 +211,8 @@ int kvflux_paged_attention_noalloc(const void* key_cache, const void* value_cach
  * query i attends to tokens [0, kv_len - query_tokens + i].
  * F16/BF16 caches: Q is rounded to the cache dtype and the softmax weights to
  * the cache dtype before the MFMA products; accumulation and softmax are
- * FP32. F32 caches: FP32 MFMAs on Q, K, V and the weights as they are (the
- * 1e-5 contract of kvflux_paged_prefill_exact, head_size 64 or 128).
+ * FP32. F32 caches: Q, K, V and the weights as three BF16 parts each (FP32
+ * accuracy; FP32 MFMAs where a value has no such parts: the 1e-5 contract of kvflux_paged_prefill_exact, head_size 64 or 128).
  * KVFLUX_ERR_UNSUPPORTED unless head_size is 64, 128 or 256 (F32: 64 or
  * 128), block_size is a power of two up to 256 and kv_len is below 2^31.
  * Any GQA group query_heads / num_kv_heads: up to 512 at head_size 64, 256 at

@@ -197,7 +197,7 @@ bool prefill_shape_ok(const PagedKVLayout& layout, std::size_t query_tokens, std
 }
 
 // The rounded (2e-2) MFMA prefill: Fast, or Auto from 16 query tokens on.
-// FP32 caches take FP32 MFMAs there, whose products are exact.
+// FP32 caches keep FP32 accuracy there (every value in three BF16 parts).
 bool prefill_eligible(const PagedKVLayout& layout, std::size_t query_tokens, std::size_t kv_len,
                       AttentionPrecision precision) {
     if (precision == AttentionPrecision::Exact) return false;
