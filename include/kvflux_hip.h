@@ -240,6 +240,13 @@ int kvflux_paged_prefill(const void* key_cache, const void* value_cache,
  * (src/v2/paged_attention.cu:108-128); the C++ paged_attention uses it. */
 int kvflux_paged_prefill_workspace_size(uint64_t num_kv_heads, uint64_t head_size, uint64_t kv_len,
                                         uint64_t query_tokens, uint64_t query_heads, size_t* bytes);
+/* What kvflux_paged_prefill_split (exact != 0: kvflux_paged_prefill_exact)
+ * launches for a call, with or without a workspace: the workgroups that share
+ * a query block's keys (key_splits) and the groups of wavefronts in one that
+ * do (key_parts). Host arithmetic only: no device is touched. */
+int kvflux_paged_prefill_plan(uint64_t num_kv_heads, uint64_t head_size, int dtype, int exact,
+                              uint64_t kv_len, uint64_t query_tokens, uint64_t query_heads,
+                              int with_workspace, uint32_t* key_splits, uint32_t* key_parts);
 int kvflux_paged_prefill_split(const void* key_cache, const void* value_cache,
                                uint64_t num_blocks, uint64_t num_kv_heads, uint64_t block_size,
                                uint64_t head_size, int dtype, const uint64_t* block_table,

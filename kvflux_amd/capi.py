@@ -19,6 +19,7 @@ DIST_UNIFORM, DIST_NORMAL = 0, 1
 
 _vp, _u64, _sz, _i32 = C.c_void_p, C.c_uint64, C.c_size_t, C.c_int
 _pu64 = C.POINTER(C.c_uint64)
+_pu32 = C.POINTER(C.c_uint32)
 _pf = C.POINTER(C.c_float)
 
 # name -> (restype, argtypes)
@@ -63,6 +64,7 @@ SIGNATURES = {
     "kvflux_paged_prefill": (_i32, [_vp, _vp, _u64, _u64, _u64, _u64, _i32, _vp, _u64, _u64,
                                     _u64, _u64, _vp, _vp, _vp]),
     "kvflux_paged_prefill_workspace_size": (_i32, [_u64, _u64, _u64, _u64, _u64, C.POINTER(_sz)]),
+    "kvflux_paged_prefill_plan": (_i32, [_u64, _u64, _i32, _i32, _u64, _u64, _u64, _i32, _pu32, _pu32]),
     "kvflux_paged_prefill_split": (_i32, [_vp, _vp, _u64, _u64, _u64, _u64, _i32, _vp, _u64, _u64,
                                           _u64, _u64, _vp, _vp, _vp, _u64, _vp]),
     "kvflux_paged_prefill_exact": (_i32, [_vp, _vp, _u64, _u64, _u64, _u64, _i32, _vp, _u64, _u64,

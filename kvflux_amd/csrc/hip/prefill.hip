@@ -717,12 +717,14 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
             lds_barrier();
             if (part == 0) {
                 const pf_f32x4_t other = red[(kDt + 1) * 64];
-                const bool mine = lazy_of[n] > -INFINITY, theirs = other[1] > -INFINITY;
-                const float a = -nref[n][0], b = -other[0];
-                const float m = mine && (!theirs || a > b) ? a : b;
-                // A half without a key of the row holds zeros (factor 1).
-                const float fa = mine ? __builtin_amdgcn_exp2f(a - m) : 1.0f;
-                const float fb = theirs ? __builtin_amdgcn_exp2f(b - m) : 1.0f;
+                // A side that has seen no score above -inf has no reference
+                // point: factor 0. With none on either side the row has no
+                // softmax (every split starts at a key all its rows see) and
+                // -inf - -inf makes it NaN, as with one key part.
+                const float a = lazy_of[n] > -INFINITY ? -nref[n][0] : -INFINITY;
+                const float b = other[1] > -INFINITY ? -other[0] : -INFINITY;
+                const float m = __builtin_elementwise_maximum(a, b);
+                const float fa = __builtin_amdgcn_exp2f(a - m), fb = __builtin_amdgcn_exp2f(b - m);
                 lsum[n] = lsum[n] * fa + red[kDt * 64] * fb;
                 nref[n][0] = -m;
 #pragma unroll
@@ -1453,6 +1455,31 @@ extern "C" int kvflux_paged_prefill_workspace_size(uint64_t num_kv_heads, uint64
     const std::uint64_t exact =
         head_size == 256 ? 0 : prefill_most_splits(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, true).workspace;
     *bytes = static_cast<size_t>(rounded > exact ? rounded : exact);
+    return KVFLUX_OK;
+}
+
+extern "C" int kvflux_paged_prefill_plan(uint64_t num_kv_heads, uint64_t head_size, int dtype, int exact,
+                                         uint64_t kv_len, uint64_t query_tokens, uint64_t query_heads,
+                                         int with_workspace, uint32_t* key_splits, uint32_t* key_parts) {
+    if (!key_splits || !key_parts) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged prefill plan: null pointer");
+    *key_splits = *key_parts = 0;
+    if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
+    if (num_kv_heads == 0 || query_heads == 0 || query_heads % num_kv_heads != 0 || query_heads > 0xffffffffULL ||
+        (head_size != 64 && head_size != 128 && head_size != 256) || kv_len == 0 || kv_len > 0x7fffffffULL ||
+        query_tokens == 0 || query_tokens > kv_len) {
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged prefill plan: invalid shape");
+    }
+    const bool f32 = dtype == KVFLUX_DTYPE_F32;
+    const bool three_parts = f32 || exact != 0;
+    const std::uint64_t group = query_heads / num_kv_heads;
+    const std::uint64_t most =
+        with_workspace
+            ? prefill_most_splits(head_size, group, num_kv_heads, kv_len, query_tokens, query_heads, three_parts).splits
+            : 1;
+    const PrefillPlan plan = prefill_choice(head_size, three_parts, f32, group, num_kv_heads, kv_len, query_tokens,
+                                            query_heads, most, true);
+    *key_splits = plan.splits;
+    *key_parts = static_cast<uint32_t>(plan.key_parts);
     return KVFLUX_OK;
 }
 

@@ -36,6 +36,14 @@ def arena(name, kv_heads, bs, head_size, kv_lens, seed):
     return kc, vc, blocks, table, width
 
 
+def plan(name, kv_heads, q_heads, head_size, kv, tq, exact=False, workspace=False):
+    """(key splits, key parts) that the call launches."""
+    splits, parts = C.c_uint32(0), C.c_uint32(0)
+    capi.check(capi.lib().kvflux_paged_prefill_plan(kv_heads, head_size, DTYPES[name][0], int(exact), kv, tq, q_heads,
+                                                    int(workspace), C.byref(splits), C.byref(parts)))
+    return splits.value, parts.value
+
+
 SHAPES = [  # name, kv heads, q heads, D, block size, (kv, queries) of each sequence
     ("BFloat16", 2, 8, 128, 16, [(1, 1), (31, 31), (33, 33), (64, 64), (65, 65)]),
     ("Float16", 1, 4, 128, 8, [(97, 97), (320, 1), (352, 40), (130, 130)]),  # rows starting in either half
@@ -109,6 +117,44 @@ def test_exact_key_parts(gpu, case):
         got = out.download(np.float32)
         assert np.all(got[q.size:] == 7.0) and np.all(np.isnan(ws.download(np.float32)[size // 4:]))
         assert np.abs(got[:q.size] - exp).max() < 1e-5
+
+
+@pytest.mark.parametrize("name,D,exact,kv", [
+    ("BFloat16", 64, False, 150), ("BFloat16", 128, False, 150), ("BFloat16", 256, False, 150),
+    ("Float16", 128, False, 150), ("BFloat16", 64, True, 640), ("BFloat16", 128, True, 200),
+])
+def test_rows_without_a_score_above_minus_infinity(gpu, name, D, exact, kv):
+    """Two key parts: the first keys score -inf for every row (their products
+    overflow; FP16: an infinite element), so the rows that see no other key
+    have no softmax and come out NaN, as with one key part; a key with a NaN
+    makes every row that sees it NaN; the rows between are the oracle's."""
+    kv_heads, q_heads, bs, none, nan = 2, 8, 16, 6, 70
+    assert plan(name, kv_heads, q_heads, D, kv, kv, exact) == (1, 2)
+    code, host = DTYPES[name]
+    kc, vc, blocks, table, width = arena(name, kv_heads, bs, D, [kv], 870 + D)
+    kh = kc.download(host).reshape(blocks, kv_heads, bs, D)
+    at = lambda t: (int(table[0, t // bs]), slice(None), t % bs)  # noqa: E731
+    for t in range(none):
+        kh[at(t)][:, 3] = 0x7c00 if name == "Float16" else 0x7f62  # inf, 3.004e38
+    q = oracle.random_elements(0, kv * q_heads * D, oracle.F32, 1, 890).reshape(kv, q_heads, D)
+    q[:, :, 3] = -40.0
+    exp = oracle.paged_attention_causal(kh.reshape(-1), vc.download(host), kv_heads, bs, D, code, table[0], kv,
+                                        q.reshape(-1), kv, q_heads, threads=8).reshape(kv, q_heads, D)
+    kh[at(nan)][:, 9] = 0x7fff
+    kc.upload(kh.reshape(-1))
+    td, qd = buffer_like(table.reshape(-1)), buffer_like(q.reshape(-1))
+    args = (kc.ptr, vc.ptr, blocks, kv_heads, bs, D, code, td.ptr, width, kv, kv, q_heads, qd.ptr)
+    out = buffer_like(np.full(q.size, 7.0, np.float32))
+    capi.check(getattr(capi.lib(), "kvflux_paged_prefill_exact" if exact else "kvflux_paged_prefill_split")(
+        *args, out.ptr, None, 0, None))
+    device.synchronize()
+    got = out.download(np.float32).reshape(kv, q_heads, D)
+    assert np.all(np.isnan(got[:none])) and np.all(np.isnan(got[nan:]))
+    assert np.abs(got[none:nan] - exp[none:nan]).max() < (1e-5 if exact else 2e-2)
+    if not exact:  # the entry without key parts
+        capi.check(capi.lib().kvflux_paged_prefill(*args, out.ptr, None))
+        device.synchronize()
+        assert np.array_equal(np.isnan(out.download(np.float32)), np.isnan(got.reshape(-1)))
 
 
 @pytest.mark.parametrize("D,bs,kv,tq", [(128, 16, 200, 200), (64, 1, 2500, 40), (128, 4, 9000, 33)])
