@@ -780,9 +780,13 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 //    accumulator dominated by one large weight, small weights lose bits in the
 //    same direction at every step: 2.8e-5 on a row of one dominant key and
 //    4095 keys 2^-25 below it).
-//  * An infinity or NaN (or a value that rounds to one in BF16) has no parts.
-//    Such a half, and every half of a wavefront with such a query row, takes
-//    the FP32 MFMAs on values read from global memory (direct_scores,
+//  * A value of 2^56 or more (an infinity or NaN among them) has no parts:
+//    below it a sum of 128 part products stays under 2^119, so none leaves
+//    FP32's range where the products of the whole values would not (a part
+//    product that overflows to +inf before one that overflows to -inf made
+//    rows NaN whose one large key FP32 products drop). A half with such a
+//    value, and every half of a wavefront with such a query row, takes the
+//    FP32 MFMAs on values read from global memory (direct_scores,
 //    direct_values).
 // Measured against v_mfma_f32_16x16x4_f32 throughout, 64-bit errors beside:
 // 4 x 384..1024 tokens, 16/4 heads 132.3 -> 93.4 us (3.3e-7 -> 2.0e-7), 813
@@ -801,6 +805,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
     constexpr int kLoads = 2 * kKeys * kCpr / kPfThreads;  // 8-value chunks per thread and half, K's before V's
     constexpr int kVSwz = kCpr / 8;
     constexpr float kLazy = M::kLazyLog2;
+    constexpr float kPartsBelow = 0x1p56f;     // values from here on take the FP32 MFMAs
     static_assert(kLoads >= 1 && 2 * kKeys * kCpr % kPfThreads == 0, "half split");
     // [buffer][K, V][part]
     __shared__ __attribute__((aligned(16))) unsigned char parts_lds[2][2][3][kPartBytes];
@@ -845,12 +850,11 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
     stage((half_begin & ~win_mask) * kKeys >> p.bs_shift);
     if (tid < 2) no_parts[tid] = 0;
 
-    // Eight values to 16 bytes of each part; false when some value has none
-    // (the last remainder is then not a number).
+    // Eight values to 16 bytes of each part; false when some value has none.
     auto split8 = [](const float4& a, const float4& b, uint4 (&out)[3]) -> bool {
         const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         std::uint32_t w[3][4];
-        float rest = 0.0f;
+        float largest = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             pf_f32x2_t v{x[2 * j], x[2 * j + 1]};
@@ -860,11 +864,11 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
                 w[i][j] = __builtin_bit_cast(std::uint32_t, h);
                 v -= __builtin_convertvector(h, pf_f32x2_t);
             }
-            rest = max3(rest, v[0], v[1]);  // propagates NaN
+            largest = max3(largest, __builtin_fabsf(x[2 * j]), __builtin_fabsf(x[2 * j + 1]));  // propagates NaN
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) out[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
-        return rest == rest;
+        return largest < kPartsBelow;
     };
     Vec qop[3][kSteps];
     bool q_parts = true;
