@@ -780,14 +780,23 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 //    accumulator dominated by one large weight, small weights lose bits in the
 //    same direction at every step: 2.8e-5 on a row of one dominant key and
 //    4095 keys 2^-25 below it).
-//  * A value of 2^56 or more (an infinity or NaN among them) has no parts:
-//    below it a sum of 128 part products stays under 2^119, so none leaves
-//    FP32's range where the products of the whole values would not (a part
-//    product that overflows to +inf before one that overflows to -inf made
-//    rows NaN whose one large key FP32 products drop). A half with such a
-//    value, and every half of a wavefront with such a query row, takes the
-//    FP32 MFMAs on values read from global memory (direct_scores,
-//    direct_values).
+//  * BF16 parts end at 2^-133 (2^-126 but for subnormals): below about 2^-110
+//    three of them are not x any more, so values under 2^-100 have none. (The
+//    magnitude is tested: the last remainder, which is 0 for all others, costs
+//    two operations more a value and measured 95.0 against 93.4 us, 4 x
+//    384..1024 tokens, 16/4 heads.)
+//    The weights are split scaled by 2^32 (undone, exactly, where the
+//    half-tile's sums reach the accumulator), so that they have theirs down to
+//    the smallest that the exponential gives.
+//  * A value of 2^56 or more (an infinity or NaN among them) has none: below
+//    it a sum of 128 part products stays under 2^119 (of 32 with weights of
+//    2^8, scaled, under 2^101), so none leaves FP32's range where the products
+//    of the whole values would not (a part product that overflows to +inf
+//    before one that overflows to -inf made rows NaN whose one large key FP32
+//    products drop).
+//  * A half with a value without parts, and every half of a wavefront with
+//    such a query row, takes the FP32 MFMAs on values read from global memory
+//    (direct_scores, direct_values).
 // Measured against v_mfma_f32_16x16x4_f32 throughout, 64-bit errors beside:
 // 4 x 384..1024 tokens, 16/4 heads 132.3 -> 93.4 us (3.3e-7 -> 2.0e-7), 813
 // tokens, 12/1 heads 63.8 -> 45.6 (4.0e-7 -> 2.5e-7), 8 x 4096 tokens, 32/8
@@ -805,7 +814,10 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
     constexpr int kLoads = 2 * kKeys * kCpr / kPfThreads;  // 8-value chunks per thread and half, K's before V's
     constexpr int kVSwz = kCpr / 8;
     constexpr float kLazy = M::kLazyLog2;
-    constexpr float kPartsBelow = 0x1p56f;     // values from here on take the FP32 MFMAs
+    // Values past these magnitudes, zeros apart, take the FP32 MFMAs.
+    constexpr std::uint32_t kPartsFromBits = (127 - 100) << 23;  // 2^-100
+    constexpr float kPartsBelow = 0x1p56f;
+    constexpr float kWeightScale = 0x1p32f;
     static_assert(kLoads >= 1 && 2 * kKeys * kCpr % kPfThreads == 0, "half split");
     // [buffer][K, V][part]
     __shared__ __attribute__((aligned(16))) unsigned char parts_lds[2][2][3][kPartBytes];
@@ -850,35 +862,39 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
     stage((half_begin & ~win_mask) * kKeys >> p.bs_shift);
     if (tid < 2) no_parts[tid] = 0;
 
-    // Eight values to 16 bytes of each part; false when some value has none.
-    auto split8 = [](const float4& a, const float4& b, uint4 (&out)[3]) -> bool {
+    // Eight values times `scale`, not rounded in between, to 16 bytes of each
+    // part; false when some value has none.
+    auto split8 = [](const float4& a, const float4& b, float scale, uint4 (&out)[3]) -> bool {
         const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         std::uint32_t w[3][4];
         float largest = 0.0f;
+        std::uint32_t smallest = 0xffffffffu;  // twice the magnitude's bits - 1: a zero is above all others
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            pf_f32x2_t v{x[2 * j], x[2 * j + 1]};
+            const pf_f32x2_t y{x[2 * j] * scale, x[2 * j + 1] * scale};
+            pf_bf16x2_t h = __builtin_convertvector(y, pf_bf16x2_t);
+            w[0][j] = __builtin_bit_cast(std::uint32_t, h);
+            const pf_f32x2_t first = __builtin_convertvector(h, pf_f32x2_t);
+            pf_f32x2_t v{fmaf(x[2 * j], scale, -first[0]), fmaf(x[2 * j + 1], scale, -first[1])};
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const pf_bf16x2_t h = __builtin_convertvector(v, pf_bf16x2_t);
+            for (int i = 1; i < 3; ++i) {
+                h = __builtin_convertvector(v, pf_bf16x2_t);
                 w[i][j] = __builtin_bit_cast(std::uint32_t, h);
                 v -= __builtin_convertvector(h, pf_f32x2_t);
             }
-            largest = max3(largest, __builtin_fabsf(x[2 * j]), __builtin_fabsf(x[2 * j + 1]));  // propagates NaN
+            largest = max3(largest, __builtin_fabsf(y[0]), __builtin_fabsf(y[1]));  // propagates NaN
+            smallest = min(smallest, min(2 * __float_as_uint(y[0]) - 1, 2 * __float_as_uint(y[1]) - 1));
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) out[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
-        return largest < kPartsBelow;
+        return largest < kPartsBelow && smallest >= 2 * kPartsFromBits - 1;
     };
     Vec qop[3][kSteps];
     bool q_parts = true;
 #pragma unroll
     for (int kk = 0; kk < kSteps; ++kk) {
-        const float4 lo = qraw[kk][0], hi = qraw[kk][1];
-        const float sc = p.scale_log2;
         uint4 w[3];
-        q_parts &= split8(make_float4(lo.x * sc, lo.y * sc, lo.z * sc, lo.w * sc),
-                          make_float4(hi.x * sc, hi.y * sc, hi.z * sc, hi.w * sc), w);
+        q_parts &= split8(qraw[kk][0], qraw[kk][1], p.scale_log2, w);
 #pragma unroll
         for (int i = 0; i < 3; ++i) qop[i][kk] = __builtin_bit_cast(Vec, w[i]);
     }
@@ -925,7 +941,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
             const int kv = e < kKeys * kCpr ? 0 : 1, row = (e / kCpr) % kKeys, c = e % kCpr;
             const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             uint4 w[3];
-            const bool ok = split8(live[i] ? held[i].lo : zero, live[i] ? held[i].hi : zero, w);
+            const bool ok = split8(live[i] ? held[i].lo : zero, live[i] ? held[i].hi : zero, 1.0f, w);
             const int at = row * kRowBytes + (c ^ (kv == 0 ? kswz(row) : vswz(row))) * 16;
 #pragma unroll
             for (int k = 0; k < 3; ++k) *reinterpret_cast<uint4*>(&parts_lds[buf][kv][k][at]) = w[k];
@@ -1054,7 +1070,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 std::uint32_t x[3];
-                M::split3(pr[2 * j], pr[2 * j + 1], x);
+                M::split3(pr[2 * j] * kWeightScale, pr[2 * j + 1] * kWeightScale, x);
 #pragma unroll
                 for (int k = 0; k < 3; ++k) w[k][j] = x[k];
             }
@@ -1076,7 +1092,7 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillPa
             large = M::mma(a[0], pb[1], large);
             small = M::mma(a[0], pb[2], small);
             large = M::mma(a[0], pb[0], large);
-            acc[dt] += large + small;
+            acc[dt] += (large + small) * (1.0f / kWeightScale);
         }
     };
 

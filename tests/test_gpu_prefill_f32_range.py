@@ -67,3 +67,47 @@ def test_finite_elements_whose_score_overflows(gpu, D, bs, kv, tq, element):
     got, exp = run(D, bs, kv, tq, 1000 + kv, change)
     assert np.all(np.isfinite(got))
     assert np.abs(got - exp).max() < 1e-5
+
+
+@pytest.mark.parametrize("D,bs,kv,tq", SHAPES)
+@pytest.mark.parametrize("power", [-100, -110, -120])
+def test_small_values(gpu, D, bs, kv, tq, power):
+    """V near 2^power: relative to it, the outputs are those of V near 1."""
+    got, exp = run(D, bs, kv, tq, 1020 + kv, lambda k, v, q: np.ldexp(v, power, out=v))
+    assert np.abs(got.astype(np.float64) - exp).max() < 1e-6 * 2.0 ** power * 4
+
+
+@pytest.mark.parametrize("D,bs,kv,tq", SHAPES)
+@pytest.mark.parametrize("power", [100, 118])
+def test_small_keys_large_queries(gpu, D, bs, kv, tq, power):
+    """K near 2^-power and Q near 2^power: the scores of both near 1."""
+    def change(k, v, q):
+        np.ldexp(k, -power, out=k)
+        np.ldexp(q, power, out=q)
+
+    got, exp = run(D, bs, kv, tq, 1040 + kv, change)
+    assert np.abs(got - exp).max() < 1e-5
+
+
+@pytest.mark.parametrize("D,bs,kv,tq", SHAPES)
+def test_small_weights(gpu, D, bs, kv, tq):
+    """A column whose only nonzero V belongs to a key of weight near 2^-121:
+    its outputs are that weight's. The queries have one nonzero dimension, so
+    its score is one product (later dimensions add exact zeros): at most four
+    roundings of values up to 128, 2^-18 each, and the query's and the scale's
+    own, 2^-24 of 121 each: (2^-16 + 242 * 2^-24) * ln 2 = 2.1e-5 of the weight."""
+    key = (kv - tq) // 2 + 2
+
+    def change(k, v, q):
+        k[:, :, 3] = 0.0
+        q[:] = 0.0
+        q[:, :, 3] = 8.0
+        k[key, :, 3] = -120.5 / 8.0 * np.sqrt(D) / 1.4427
+        v[:, :, 7] = 0.0
+        v[key, :, 7] = 1.2345678 * 2.0 ** 20
+
+    got, exp = run(D, bs, kv, tq, 1060 + kv, change)
+    rows = slice(max(0, key + 1 - (kv - tq)), None)
+    assert np.abs(exp[rows, :, 7]).min() > 2.0 ** -126
+    assert np.abs(got[rows, :, 7] / exp[rows, :, 7].astype(np.float64) - 1).max() < 3e-5
+    assert np.abs(got - exp).max() < 1e-5
