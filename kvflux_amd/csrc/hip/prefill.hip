@@ -766,9 +766,10 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 // FP32 caches: the exact variant's plan with K and V in three BF16 parts as
 // well. v_mfma_f32_16x16x4_f32 runs at a sixteenth of the BF16 rate, and a
 // kernel on it is bound by it (124 of 157 TFLOP/s, 8.4 us per 128 rows x 64
-// keys); with x = hi + mid + lo (8 bits each, exact) a product is the six part
-// products down to 2^-18 of it, the three dropped ones being under 2^-26, less
-// than half the rounding of one FP32 product: six BF16 MFMAs for 32 dims in
+// keys); with x = hi + mid + lo (8 bits each, exact; |mid| <= 2^-8 |x|, |lo| <=
+// 2^-17 |x|) a product is six part products. The three left out (mid lo, lo mid
+// and lo lo) are at most 2^-24 of it, one FP32 rounding of a product, which the
+// FP32 MFMA makes at every addition as well: six BF16 MFMAs for 32 dims in
 // place of eight FP32 ones of twice the time each.
 //  * The parts of a half-tile (32 keys) are made once per workgroup, on the
 //    way from global memory (registers, one half ahead of its use) to LDS, and

@@ -1,4 +1,5 @@
-"""CPU emulation of the exact attention kernels' FP16 weight path.
+"""CPU emulation of the exact attention kernels' splits: the FP16 weight path
+(first), the FP32 prefill's BF16 parts (last).
 
 The exact kernels (prefill.hip PfF16Exact, attention.hip on FP16 caches) feed
 the softmax weights to FP16 MFMAs as three FP16 parts and divide by an FP32
@@ -58,3 +59,38 @@ def test_f16_weight_split_emulation():
     assert abs(unscaled - exact) > 1e-5
     assert abs(plain_sum - exact) > 1e-5
     assert abs(scaled - exact) < 1e-6
+
+
+def split3_bf16(x):
+    """The FP32 prefill's three BF16 parts of x (FP32), as float64 arrays."""
+    parts, r = [], np.asarray(x, np.float32)
+    for _ in range(3):
+        bits = r.view(np.uint32).astype(np.uint64)
+        up = bits + np.uint64(0x7fff) + ((bits >> np.uint64(16)) & np.uint64(1))  # nearest, ties to even
+        h = (up & np.uint64(0xffff0000)).astype(np.uint32).view(np.float32)
+        parts.append(h.astype(np.float64))
+        r = r - h  # exact
+    return parts, r
+
+
+def test_bf16_parts_and_the_products_left_out():
+    """Three BF16 parts are x exactly (values of 2^-100 and more; 2^23 mantissas
+    at both ends of the range that has parts), |mid| <= 2^-8 |x| and |lo| <=
+    2^-17 |x|. So the products that the FP32 prefill leaves out, mid lo + lo mid
+    + lo lo, are at most 2^-24 (1 + 2^-10) of a product: one rounding of it,
+    which single mantissas come close to."""
+    x = (np.arange(1 << 23, dtype=np.uint32) | np.uint32(127 << 23)).view(np.float32)
+    for power in (-100, 0, 55):
+        y = np.ldexp(x, power)
+        (hi, mid, lo), rest = split3_bf16(y)
+        assert not rest.any() and np.array_equal(hi + mid + lo, y.astype(np.float64))
+    (hi, mid, lo), _ = split3_bf16(x)
+    x = x.astype(np.float64)
+    assert np.abs(mid / x).max() <= 2.0**-8 and np.abs(lo / x).max() <= 2.0**-17
+    squares = np.abs(2 * mid * lo + lo * lo) / (x * x)  # of x x
+    assert 2.0**-24.1 < squares.max() <= 2.0**-24 * (1 + 2.0**-10)
+    rng = np.random.default_rng(7)
+    other = rng.permutation(len(x))
+    left_out = np.abs(mid * lo[other] + lo * mid[other] + lo * lo[other]) / (x * x[other])
+    assert left_out.max() <= 2.0**-24 * (1 + 2.0**-10)
+    assert np.sqrt((squares**2).mean()) < 2.0**-26.5  # over all mantissas

@@ -111,3 +111,20 @@ def test_small_weights(gpu, D, bs, kv, tq):
     assert np.abs(exp[rows, :, 7]).min() > 2.0 ** -126
     assert np.abs(got[rows, :, 7] / exp[rows, :, 7].astype(np.float64) - 1).max() < 3e-5
     assert np.abs(got - exp).max() < 1e-5
+
+
+@pytest.mark.parametrize("D,bs,kv,tq", SHAPES)
+def test_mantissas_that_lose_most(gpu, D, bs, kv, tq):
+    """K, Q and V of the mantissa whose part products left out weigh most
+    (2^-24 of a product) at random signs and powers of two: the scores move by
+    at most 2^-24 * sum |q k| / sqrt(D) <= 2^-24 sqrt(D) * 2.3, the outputs by
+    that and a rounding of each: under 2e-6, the sums' own roundings aside."""
+    rng = np.random.default_rng(kv)
+
+    def change(k, v, q):
+        for x in (k, v, q):
+            x[:] = rng.choice([-1.0, 1.0], x.shape) * np.float32(1.0038986) * np.exp2(-rng.integers(0, 3, x.shape))
+
+    got, exp = run(D, bs, kv, tq, 1080 + kv, change)
+    assert np.abs(got - exp).max() < 1e-5
+    assert np.sqrt(((got - exp).astype(np.float64) ** 2).mean()) < 1e-6
