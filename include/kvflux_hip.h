@@ -182,6 +182,16 @@ int kvflux_paged_attention(const void* key_cache, const void* value_cache,
                            const float* query, float* output, void* workspace,
                            size_t workspace_bytes, void* stream);
 
+/* What kvflux_paged_attention launches on the current device for a batch call
+ * (seq_lens != NULL) with workspace_bytes of workspace: query heads per work
+ * item, heads of a second launch for those past the last whole set (0: one
+ * launch), the least tokens of an item, and the partial slots of a (row, head)
+ * (0: no partials and no combine launch). For tests and tools. */
+int kvflux_paged_attention_plan(uint64_t num_kv_heads, uint64_t block_size, uint64_t head_size, int dtype,
+                                uint64_t kv_len, uint64_t num_rows, uint64_t query_heads,
+                                uint64_t workspace_bytes, uint32_t* heads_per_item, uint32_t* heads_rest,
+                                uint32_t* item_tokens, uint32_t* partial_slots);
+
 /* kvflux_paged_attention_noalloc: kvflux_paged_attention without a workspace
  * argument and without any device allocation, for callers that cannot
  * allocate (code under HIP graph capture, serving loops that forbid

@@ -1700,6 +1700,12 @@ int resident_slots_for(std::uint32_t sub, int* out) {
     }
 }
 
+// Resident workgroups of the block-size-16 kernel on items of `sub` heads.
+template <typename E, int kD>
+int bs16_slots(bool small, std::uint32_t sub, int* out) {
+    return small ? resident_slots_for<E, kD, true>(sub, out) : resident_slots_for<E, kD, false>(sub, out);
+}
+
 // log2 of a power of two.
 inline std::uint32_t log2_pow2(std::uint64_t x) {
     std::uint32_t l = 0;
@@ -1817,28 +1823,39 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             // 8, say) takes sets of 16 (or 8) heads plus one launch for the
             // heads past the last set, rather than many narrow sets.
             std::uint32_t rest = 0;
+            int rest_slots = 0;
             if (!small && kD != 256 && g > 8 && sub < 4) {
                 sub = g > 16 && g % 16 <= 8 ? 16u : 8u;
                 rest = g % sub;
-            } else if ((small || kD == 256) && g > cap && sub < 4) {
-                // The same for the shapes of at most `cap` heads an item: sets of
-                // that many and the rest (24 rows of U[500, 12000] tokens, 28/4
-                // heads, as seven sets of one head and as 5 + 2: 8-token pages
-                // at 128 197.8 and 99.5 us, head size 256 366 and 189).
-                sub = cap;
-                rest = g % sub;
+            } else if ((small || kD == 256) && g > cap && sub < 4 && g / sub >= g / cap + 3) {
+                // The same for the shapes of at most `cap` heads an item, where it
+                // saves two sets or more (the second launch reads the pages from
+                // HBM again: 64 rows of U[4000, 16000] tokens, 4 kv heads, head
+                // size 256, one launch and two: group 6 as 2 x 3 and 5 + 1 604
+                // and 778 us, group 9 as 3 x 3 and 5 + 4 845 and 792, group 7 as
+                // 7 x 1 and 5 + 2 1707 and 783, group 14 as 7 x 2 and 2 x 5 + 4
+                // 1718 and 1021; 8-token pages at 128 330 and 429, 440 and 436,
+                // 824 and 430, 825 and 560) and one launch would take the grid
+                // more rounds of 512-token items than two (4 rows of 300 to 2000
+                // tokens, 1 kv head, group 11, 64, 128 and 256: 15.2 and 20.1,
+                // 18.7 and 22.6, 22.5 and 27.8 us).
+                int narrow = 0, wide = 0;
+                int st = bs16_slots<E, kD>(small, sub, &narrow);
+                if (st == KVFLUX_OK) st = bs16_slots<E, kD>(small, cap, &wide);
+                if (st == KVFLUX_OK) st = bs16_slots<E, kD>(small, g % cap, &rest_slots);
+                if (st != KVFLUX_OK) return st;
+                const std::uint64_t items = rows * max_chunks * p.heads;
+                auto rounds = [](std::uint64_t n, int slots) { return (n + slots - 1) / slots; };
+                if (rounds(items * (g / sub), narrow) > rounds(items * (g / cap), wide) + rounds(items, rest_slots)) {
+                    sub = cap;
+                    rest = g % sub;
+                }
             }
             const std::uint64_t sets = g / sub;  // head sets per kv head, each its own work items
             if (2 * rows * max_chunks * p.heads * sets > 0xffffffffULL) return plan_fallback(kD, group, max_chunks, plan);
-            int rest_slots = 0;
-            if (rest > 0) {
-                const int st = small ? resident_slots_for<E, kD, true>(rest, &rest_slots)
-                                     : resident_slots_for<E, kD, false>(rest, &rest_slots);
-                if (st != KVFLUX_OK) return st;
-            }
             int slots = 0;
-            int status = KVFLUX_OK;
-            status = small ? resident_slots_for<E, kD, true>(sub, &slots) : resident_slots_for<E, kD, false>(sub, &slots);
+            int status = bs16_slots<E, kD>(small, sub, &slots);
+            if (status == KVFLUX_OK && rest > 0) status = bs16_slots<E, kD>(small, rest, &rest_slots);
             if (status != KVFLUX_OK) return status;
             // Work item size: the largest chunk (up to 4096 tokens, less for
             // small pages) that still gives at least 8 items per resident
@@ -2083,23 +2100,10 @@ bool uses_split(std::uint64_t head_dim, std::uint64_t group) {
     return (head_dim == 64 || head_dim == 128 || head_dim == 256 || head_dim == 96 || head_dim == 80) && group >= 1;
 }
 
-// Argument checks shared by both entry points; fills `p` and `plan`.
-// scratch_bytes: what the caller has for the partials.
-int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks, uint64_t num_kv_heads,
-            uint64_t block_size, uint64_t head_size, int dtype, const uint64_t* block_table,
-            uint64_t max_blocks_per_seq, const uint64_t* seq_lens, uint64_t kv_len, uint64_t num_rows,
-            uint64_t query_heads, const float* query, float* output, uint64_t scratch_bytes, Params* p, Plan* plan) {
-    if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
-    if (!key_cache || !value_cache || !block_table || !query || !output) {
-        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: null pointer");
-    }
-    if (num_blocks == 0 || num_kv_heads == 0 || block_size == 0 || head_size == 0 ||
-        query_heads == 0 || query_heads % num_kv_heads != 0) {
-        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: invalid shape");
-    }
-    if (!seq_lens && num_rows > kv_len) {
-        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: more queries than tokens");
-    }
+// The shape's part of `p` and the plan; scratch_bytes: what the caller has for
+// the partials.
+int plan_shape(uint64_t num_kv_heads, uint64_t block_size, uint64_t head_size, int dtype, uint64_t max_blocks_per_seq,
+               uint64_t kv_len, uint64_t num_rows, uint64_t query_heads, uint64_t scratch_bytes, Params* p, Plan* plan) {
     if (num_rows > 0xffffffffULL || query_heads > 0xffffffffULL || num_kv_heads > 65535 ||
         block_size > 0xffffffffULL || kv_len > 0xffffffffULL) {
         return fail(KVFLUX_ERR_UNSUPPORTED, "paged attention: dimension too large");
@@ -2111,19 +2115,12 @@ int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks,
     }
     const std::uint64_t max_chunks = (kv_len + kChunk - 1) / kChunk;
     *p = Params{};
-    p->key_cache = key_cache;
-    p->value_cache = value_cache;
-    p->num_blocks = num_blocks;
     p->heads = static_cast<std::uint32_t>(num_kv_heads);
     p->block_size = FastDiv(static_cast<std::uint32_t>(block_size));
-    p->table = block_table;
     p->width = max_blocks_per_seq;
-    p->seq_lens = seq_lens;
     p->kv_len = kv_len;
     p->num_rows = static_cast<std::uint32_t>(num_rows);
     p->query_heads = static_cast<std::uint32_t>(query_heads);
-    p->query = query;
-    p->output = output;
     p->q_group = static_cast<std::uint32_t>(group);
     p->q_first = 0;
     p->q_sets = 1;
@@ -2140,6 +2137,35 @@ int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks,
     // The partial arrays' stride; 1 (or 0) tells the kernels that no
     // partials are written.
     p->max_chunks = static_cast<std::uint32_t>(plan->chunks);
+    return KVFLUX_OK;
+}
+
+// Argument checks shared by both entry points; fills `p` and `plan`.
+int prepare(const void* key_cache, const void* value_cache, uint64_t num_blocks, uint64_t num_kv_heads,
+            uint64_t block_size, uint64_t head_size, int dtype, const uint64_t* block_table,
+            uint64_t max_blocks_per_seq, const uint64_t* seq_lens, uint64_t kv_len, uint64_t num_rows,
+            uint64_t query_heads, const float* query, float* output, uint64_t scratch_bytes, Params* p, Plan* plan) {
+    if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
+    if (!key_cache || !value_cache || !block_table || !query || !output) {
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: null pointer");
+    }
+    if (num_blocks == 0 || num_kv_heads == 0 || block_size == 0 || head_size == 0 ||
+        query_heads == 0 || query_heads % num_kv_heads != 0) {
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: invalid shape");
+    }
+    if (!seq_lens && num_rows > kv_len) {
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention: more queries than tokens");
+    }
+    const int status = plan_shape(num_kv_heads, block_size, head_size, dtype, max_blocks_per_seq, kv_len, num_rows,
+                                  query_heads, scratch_bytes, p, plan);
+    if (status != KVFLUX_OK) return status;
+    p->key_cache = key_cache;
+    p->value_cache = value_cache;
+    p->num_blocks = num_blocks;
+    p->table = block_table;
+    p->seq_lens = seq_lens;
+    p->query = query;
+    p->output = output;
     return KVFLUX_OK;
 }
 
@@ -2193,6 +2219,28 @@ extern "C" int kvflux_paged_attention_workspace_size(uint64_t num_rows, uint64_t
     if (status != KVFLUX_OK) return status;
     const std::uint64_t fine = fine_items(num_rows, kv_len, num_kv_heads, query_heads, block_size, head_size);
     if (fine > *bytes) *bytes = fine;
+    return KVFLUX_OK;
+}
+
+extern "C" int kvflux_paged_attention_plan(uint64_t num_kv_heads, uint64_t block_size, uint64_t head_size, int dtype,
+                                           uint64_t kv_len, uint64_t num_rows, uint64_t query_heads,
+                                           uint64_t workspace_bytes, uint32_t* heads_per_item, uint32_t* heads_rest,
+                                           uint32_t* item_tokens, uint32_t* partial_slots) {
+    if (!heads_per_item || !heads_rest || !item_tokens || !partial_slots)
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention plan: null pointer");
+    *heads_per_item = *heads_rest = *item_tokens = *partial_slots = 0;
+    if (dtype_bytes(dtype) == 0) return fail(KVFLUX_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
+    if (num_kv_heads == 0 || block_size == 0 || head_size == 0 || query_heads == 0 || query_heads % num_kv_heads != 0)
+        return fail(KVFLUX_ERR_INVALID_ARGUMENT, "paged attention plan: invalid shape");
+    Params p;
+    Plan plan;
+    const int status = plan_shape(num_kv_heads, block_size, head_size, dtype, kv_len / block_size + 1, kv_len, num_rows,
+                                  query_heads, workspace_bytes, &p, &plan);
+    if (status != KVFLUX_OK) return status;
+    *heads_per_item = plan.family == Family::Generic ? 1 : plan.sub;
+    *heads_rest = plan.rest;
+    *item_tokens = plan.family == Family::Bs16 ? plan.item : plan.family == Family::Split ? kChunk : 0;
+    *partial_slots = plan.chunks > 1 ? static_cast<uint32_t>(plan.chunks) : 0;
     return KVFLUX_OK;
 }
 

@@ -30,6 +30,14 @@ def least_bytes(rows, kv_len, q_heads, block_size, head_size):
     return up(rows * q_heads * chunks * head_size * 4) + up(rows * q_heads * chunks * 8)
 
 
+def plan(name, H, Hq, D, bs, rows, kv_len, workspace=1 << 40):
+    """(heads per item, heads of a second launch, least item tokens, partial slots)."""
+    found = [C.c_uint32(0) for _ in range(4)]
+    capi.check(capi.lib().kvflux_paged_attention_plan(H, bs, D, DTYPES[name][0], kv_len, rows, Hq, workspace,
+                                                      *map(C.byref, found)))
+    return tuple(x.value for x in found)
+
+
 CASES = [
     # dtype, kv heads, q heads, D, block size, lengths
     ("BFloat16", 8, 32, 128, 16, [127, 128, 129, 1500]),
@@ -95,3 +103,18 @@ def test_item_sizes(gpu, case):
         status = lib.kvflux_paged_attention(kc.ptr, vc.ptr, P, H, bs, D, code, td.ptr, width, ld.ptr, max_len, rows,
                                             Hq, qd.ptr, qd.ptr, td.ptr, least - 1, None)
         assert status == 1  # KVFLUX_ERR_INVALID_ARGUMENT, before any launch
+
+
+@pytest.mark.parametrize("name,bs,D,cap", [("BFloat16", 16, 256, 5), ("Float16", 8, 128, 5), ("BFloat16", 4, 64, 8),
+                                           ("Float32", 8, 128, 8)])
+def test_second_launch_only_where_it_saves_head_sets(gpu, name, bs, D, cap):
+    """Heads past the last set of `cap` take a launch of their own where that
+    saves two sets and the grid is filled; else the sets of the largest divisor
+    run in one launch (they share the pages in L2)."""
+    for group in range(1, 40):
+        sub = next(d for d in range(min(group, cap), 0, -1) if group % d == 0)
+        few = plan(name, 1, group, D, bs, 2, 300)
+        many = plan(name, 4, 4 * group, D, bs, 64, 16000)
+        assert few[:2] == (sub, 0)
+        saves = group > cap and sub < 4 and group // sub >= group // cap + 3
+        assert many[:2] == ((cap, group % cap) if saves else (sub, 0)), group
