@@ -165,10 +165,15 @@ int kvflux_gather_paged_kv_live(const void* key_cache, const void* value_cache,
  * to 256 rows chooses the size on the device, from seq_lens, that spreads the
  * work evenly. The least workspace accepted holds 512-token splits (256 at
  * block_size 1); for small calls kvflux_paged_attention_workspace_size gives
- * more, with which splits go down to 128 tokens. Any group is accepted (num_rows and
- * kv_len below 2^32, at most 65535 kv heads); shapes outside these take the
- * split kernel (head_size 64/80/96/128/256) or a generic kernel (any other
- * head_size up to 512).
+ * more, with which splits go down to 128 tokens. Rows of at most 512 tokens
+ * (kv_len) take one launch and no workspace, unless a workspace of the
+ * documented size is there and 128-token splits pay for the combine (FP32
+ * caches and head_size 256, a few rows of 300 tokens and more). As the split
+ * size follows from all rows' lengths and from the workspace, a row's bits may
+ * differ between batches; the same call gives the same bits. Any group is
+ * accepted (num_rows and kv_len below 2^32, at most 65535 kv heads); shapes
+ * outside these take the split kernel (head_size 64/80/96/128/256) or a generic
+ * kernel (any other head_size up to 512).
  * ------------------------------------------------------------------------- */
 int kvflux_paged_attention_workspace_size(uint64_t num_rows, uint64_t kv_len,
                                           uint64_t num_kv_heads, uint64_t query_heads,
@@ -198,7 +203,8 @@ int kvflux_paged_attention_plan(uint64_t num_kv_heads, uint64_t block_size, uint
  * hipMalloc, harnesses with a fixed memory budget). No counterpart in the
  * reference, whose paged_attention_batch allocates its metadata per call
  * (src/v2/paged_attention.cu:287-292). Same kernels, same results (bit for
- * bit) as kvflux_paged_attention. The chunk partials live in a static device
+ * bit) as kvflux_paged_attention with a workspace of the size that
+ * kvflux_paged_attention_workspace_size gives. The chunk partials live in a static device
  * array of KVFLUX_NOALLOC_SCRATCH_BYTES that each device holds until the
  * process ends; a call whose partials exceed it fails with
  * KVFLUX_ERR_UNSUPPORTED (at the 128-row, 32K-token, 32 q-head, head_size 128

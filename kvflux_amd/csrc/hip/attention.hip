@@ -1740,7 +1740,8 @@ PartialLayout partial_layout(std::uint64_t rows, std::uint64_t query_heads, std:
     return out;
 }
 
-// Small calls may take items down to kFineItem tokens: where 512-token items
+// Small calls may take items down to kFineItem tokens (rows that one item
+// covers only where that pays for the combine: plan_group): where 512-token items
 // would be at most kFineItems (about two per resident workgroup, so that
 // rounding to whole items leaves workgroups idle or waiting for one long
 // item) and the partials stay within kFineBytes (a quarter of the
@@ -1757,6 +1758,18 @@ inline std::uint64_t fine_items(std::uint64_t rows, std::uint64_t kv_len, std::u
     if (rows * heads * ((kv_len + kChunk - 1) / kChunk) > kFineItems || query_heads > kFineBytes) return 0;
     const std::uint64_t bytes = partial_layout(rows, query_heads, (kv_len + kFineItem - 1) / kFineItem, head_size).total;
     return bytes <= kFineBytes ? bytes : 0;
+}
+
+// The combine launch of a small call in tokens of an item's walk: about 4.6 us
+// (its latency, two round trips, and the launch gap) over the time of a token,
+// which grows with the head size and is larger on FP32 caches (whole FP32
+// rows in registers) and small pages. From one row of 512 tokens as one item
+// against four of 128 and the combine: 9.2 and 10.4 us at head size 64, 11.0
+// and 12.4 at 128, 18.0 and 15.7 at 256, FP32 13.0 and 12.1 at 64, 19.7 and 15.7
+// at 128. A grid that the small items fill pays up to twice that (12 rows,
+// 32/8 heads: 10.9 and 12.7 at 64, FP32 14.8 and 15.9).
+inline double combine_tokens(int head_size, bool f32, bool small_pages) {
+    return (f32 ? 33300.0 / (40 + head_size) : 92000.0 / (106 + head_size)) / (small_pages ? 1.2 : 1.0);
 }
 
 // The VALU kernels: split at head_size 64/128/256, as launches of the
@@ -1870,14 +1883,27 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             // Up to kAdaptRows rows the kernel, which knows the lengths,
             // takes the size from there on that balances the grid best.
             std::uint32_t item = 1u << shift, item_max;
-            const std::uint64_t fine = fine_items(rows, p.kv_len, p.heads, p.query_heads, bs, kD);
-            if (fine > 0 && scratch_bytes >= fine && kFineItem < item) item = kFineItem;
             // Rows of one item at most need no partials: the item is as long
             // as the longest may be, in whole steps (an item loads and masks
             // all its tiles: 100 rows of 10-80 tokens in 512-token items
             // 29.6 us, in 128-token items 14.8; one row of 30: 12.0 and 7.6).
-            const bool whole_rows = p.kv_len < item;
-            if (whole_rows) item = p.kv_len <= kItemStep ? kItemStep : static_cast<std::uint32_t>(p.kv_len + kItemStep - 1) / kItemStep * kItemStep;
+            const std::uint64_t whole = p.kv_len <= kItemStep ? kItemStep : (p.kv_len + kItemStep - 1) / kItemStep * kItemStep;
+            bool whole_rows = p.kv_len <= item;
+            const std::uint64_t fine = fine_items(rows, p.kv_len, p.heads, p.query_heads, bs, kD);
+            if (fine > 0 && scratch_bytes >= fine && kFineItem < item) {
+                const std::uint64_t per_row = rows * p.heads, parts = (p.kv_len + kFineItem - 1) / kFineItem;
+                auto rounds = [&](std::uint64_t n) {
+                    return (per_row * sets * n + slots - 1) / slots +
+                           (rest > 0 ? (per_row * n + rest_slots - 1) / rest_slots : 0);
+                };
+                const double combine = combine_tokens(kD, kF32Cache, small) * (1.0 + per_row * sets * parts / 1024.0);
+                if (!whole_rows || static_cast<double>(rounds(1) * (whole + kItemCost)) >
+                                       static_cast<double>(rounds(parts) * (kFineItem + kItemCost)) + combine) {
+                    item = kFineItem;
+                    whole_rows = false;
+                }
+            }
+            if (whole_rows) item = static_cast<std::uint32_t>(whole);
             const std::uint64_t chunks = (p.kv_len + item - 1) / item;
             const std::uint64_t items = rows * chunks * p.heads * sets;  // upper bound of the real count
             item_max = !whole_rows && rows <= kAdaptRows && items <= 0x7fffffffULL ? 1u << max_item_shift(bs) : item;

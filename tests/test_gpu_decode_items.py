@@ -105,6 +105,48 @@ def test_item_sizes(gpu, case):
         assert status == 1  # KVFLUX_ERR_INVALID_ARGUMENT, before any launch
 
 
+@pytest.mark.parametrize("name,H,Hq,D,bs", [("BFloat16", 8, 32, 128, 16), ("Float16", 2, 16, 128, 16),
+                                             ("BFloat16", 8, 64, 64, 8), ("Float32", 8, 32, 128, 16),
+                                             ("BFloat16", 4, 28, 256, 16)])
+def test_short_rows_in_one_launch(gpu, name, H, Hq, D, bs):
+    """Rows that one 512-token item covers: one launch without partials where
+    the combine would cost more than it saves (16-bit caches up to head size
+    128: everywhere), the workspace left as it is."""
+    lib, code, host = capi.lib(), *DTYPES[name]
+    for rows, kv_len in ((1, 130), (1, 256), (8, 400), (32, 512), (100, 300)):
+        _, _, item, slots = plan(name, H, Hq, D, bs, rows, kv_len)
+        may_split = name == "Float32" or D == 256
+        if not may_split or kv_len <= 256 or rows >= 32:
+            assert (item, slots) == (-(-kv_len // 128) * 128, 0), (rows, kv_len)
+        assert plan(name, H, Hq, D, bs, rows, kv_len, 0)[3] == 0  # nothing without a workspace
+        P = rows * -(-kv_len // bs)
+        kc = device.DeviceBuffer(P * H * bs * D * np.dtype(host).itemsize)
+        vc = device.DeviceBuffer(P * H * bs * D * np.dtype(host).itemsize)
+        device.fill_random(kc.ptr, P * H * bs * D, code, 1, 7)
+        device.fill_random(vc.ptr, P * H * bs * D, code, 1, 8)
+        lens = np.array([1 + (kv_len - 1) * (r + 1) // rows for r in range(rows)], np.uint64)
+        table = np.arange(P, dtype=np.uint64).reshape(rows, -1)
+        q = oracle.random_elements(0, rows * Hq * D, oracle.F32, 1, 9)
+        td, ld, qd = buffer_like(table.reshape(-1)), buffer_like(lens), buffer_like(q)
+        full = C.c_size_t(0)
+        capi.check(lib.kvflux_paged_attention_workspace_size(rows, kv_len, H, Hq, bs, D, C.byref(full)))
+        outs = []
+        for size in (full.value, 0):
+            ws, od = buffer_like(np.full(size // 4 + 64, 5.0, np.float32)), buffer_like(np.zeros(q.size, np.float32))
+            capi.check(lib.kvflux_paged_attention(kc.ptr, vc.ptr, P, H, bs, D, code, td.ptr, table.shape[1], ld.ptr,
+                                                  kv_len, rows, Hq, qd.ptr, od.ptr, ws.ptr if size else None, size,
+                                                  None))
+            device.synchronize()
+            outs.append(od.download(np.float32))
+            if slots == 0:
+                assert np.all(ws.download(np.float32) == 5.0)
+        exp = oracle.paged_attention_rows(kc.download(host), vc.download(host), H, bs, D, code, table.reshape(-1),
+                                          table.shape[1], lens, q, Hq, threads=8)
+        assert max(np.abs(out - exp).max() for out in outs) < TOL
+        if slots == 0:
+            assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("name,bs,D,cap", [("BFloat16", 16, 256, 5), ("Float16", 8, 128, 5), ("BFloat16", 4, 64, 8),
                                            ("Float32", 8, 128, 8)])
 def test_second_launch_only_where_it_saves_head_sets(gpu, name, bs, D, cap):
