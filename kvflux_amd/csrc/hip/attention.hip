@@ -1407,24 +1407,32 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
 }
 
 // Combines the chunk partials of every (row, query head) with more than one
-// chunk. One 256-thread block per (row, query head): a thread holds four dims
-// (lane d4 of a group of head_dim / 4 lanes) of the chunks g, g + groups, ...
-// of its group g, with the first two chunks' loads sent out before the chunk
-// count and weights are known, and the groups are added in order through LDS.
-// Every sum has a fixed order, so results are deterministic. The work is
-// latency: the loads of all chunks are in flight at once instead of eight at a
-// time (2 rows of 137 chunks, 32 heads: 9.6 us with 128 threads walking the
-// chunks; 4.2 us now, with 31; 16 rows of 13 chunks, 28 heads: 5.3 -> 4.0 us).
+// chunk. One block per (row, query head): a thread holds four dims (lane d4 of
+// a group of head_dim / 4 lanes) of the chunks g, g + groups, ... of its group g,
+// and the groups are added in order through LDS. Every sum has a fixed order,
+// so results are deterministic.
+// Small launches are latency: 256 threads, the loads of all chunks in flight
+// at once, the first two of a group before the chunk count is known (kAhead; 2
+// rows of 137 chunks, 32 heads: 9.6 us with 128 threads walking the chunks eight
+// at a time; 4.2 us now, with 31; 16 rows of 13 chunks, 28 heads: 5.3 -> 4.0 us).
+// Launches of more than kCombineAhead blocks, about what the chip holds at
+// once, hide that latency behind each other: there a block is one wavefront,
+// and rows without partials are dropped by their lengths before any load (250
+// rows of U[1, 700] tokens, 64/8 heads: 16.1 us with 256 threads and loads
+// ahead, 6.9 now; 250 of U[1, 3000], 32/8: 14.3 and 7.2; 128 of U[1024, 16000]:
+// 7.8 and 4.8).
 // chunk_tokens == 0: the count is the place of the first kListEnd
-// (paged_decode_bs16_kernel), else it follows from the row's length.
+// (paged_decode_bs16_kernel with a choice of item sizes), else it follows from
+// the row's length.
 // The caller's output and workspace are only known to be float-aligned.
 struct Float2 { float x, y; };
 struct Float4 { float x, y, z, w; };
-constexpr int kCombineThreads = 256;
-constexpr int kCombineWaves = kCombineThreads / 64;
+constexpr std::uint64_t kCombineAhead = 2048;
 
+template <int kCombineThreads, bool kAhead>
 __global__ __launch_bounds__(kCombineThreads) void paged_attention_combine_kernel(Params p, std::uint32_t head_dim,
                                                                                    std::uint32_t chunk_tokens) {
+    constexpr int kCombineWaves = kCombineThreads / 64;
     __shared__ float weight[kCombineThreads];
     __shared__ float wave_value[2][kCombineWaves];
     __shared__ std::uint32_t wave_end[kCombineWaves];
@@ -1446,8 +1454,13 @@ __global__ __launch_bounds__(kCombineThreads) void paged_attention_combine_kerne
         const std::uint32_t safe = c < p.max_chunks ? c : p.max_chunks - 1;
         return *reinterpret_cast<const Float4*>(acc + static_cast<std::uint64_t>(safe) * head_dim + 4 * d4);
     };
+    if (!kAhead && row_length(p, row) <= (chunk_tokens != 0 ? chunk_tokens : p.item_tokens)) return;  // uniform
     const Float2 first = *reinterpret_cast<const Float2*>(ml + 2 * (tid < p.max_chunks ? tid : p.max_chunks - 1));
-    const Float4 ahead0 = part(group), ahead1 = part(group + groups);
+    Float4 part0, part1;
+    if (kAhead) {
+        part0 = part(group);
+        part1 = part(group + groups);
+    }
 
     std::uint32_t nchunks;
     if (chunk_tokens == 0) {
@@ -1470,6 +1483,10 @@ __global__ __launch_bounds__(kCombineThreads) void paged_attention_combine_kerne
         nchunks = needed < p.max_chunks ? static_cast<std::uint32_t>(needed) : p.max_chunks;
     }
     if (nchunks == 0 || (chunk_tokens != 0 && nchunks == 1)) return;  // uniform: the row has no partials
+    if (!kAhead) {
+        part0 = part(group);
+        part1 = part(group + groups);
+    }
 
     float m = tid < nchunks ? first.x : -INFINITY;
     for (std::uint32_t c = tid + kCombineThreads; c < nchunks; c += kCombineThreads) m = fmaxf(m, ml[2 * c]);
@@ -1501,9 +1518,9 @@ __global__ __launch_bounds__(kCombineThreads) void paged_attention_combine_kerne
         if (active) {
             std::uint32_t c = group;
             if (c0 == 0) {
-                if (c < n) add(ahead0, weight[c]);
+                if (c < n) add(part0, weight[c]);
                 c += groups;
-                if (c < n) add(ahead1, weight[c]);
+                if (c < n) add(part1, weight[c]);
                 c += groups;
             }
             for (; c + 3 * groups < n; c += 4 * groups) {
@@ -1940,14 +1957,23 @@ int plan_call(const Params& p, std::uint64_t rows, std::uint64_t head_dim, std::
     return KVFLUX_OK;
 }
 
+// The rows p.row_base .. + rows.
+int launch_combine_slice(const Params& p, std::uint64_t rows, std::uint32_t head_dim, std::uint32_t chunk_tokens,
+                         hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(rows * p.query_heads));
+    if (rows * p.query_heads <= kCombineAhead)
+        hipLaunchKernelGGL((paged_attention_combine_kernel<256, true>), grid, dim3(256), 0, s, p, head_dim, chunk_tokens);
+    else
+        hipLaunchKernelGGL((paged_attention_combine_kernel<64, false>), grid, dim3(64), 0, s, p, head_dim, chunk_tokens);
+    return launch_status("paged_attention_combine_kernel");
+}
+
 int launch_combine(Params p, std::uint32_t head_dim, std::uint32_t chunk_tokens, hipStream_t s) {
     const std::uint64_t per_launch = 0x7fffffffULL / p.query_heads;
     for (std::uint64_t base = 0; base < p.num_rows; base += per_launch) {
         const std::uint64_t n = p.num_rows - base < per_launch ? p.num_rows - base : per_launch;
         p.row_base = static_cast<std::uint32_t>(base);
-        hipLaunchKernelGGL(paged_attention_combine_kernel, dim3(static_cast<unsigned>(n * p.query_heads)),
-                           dim3(kCombineThreads), 0, s, p, head_dim, chunk_tokens);
-        const int status = launch_status("paged_attention_combine_kernel");
+        const int status = launch_combine_slice(p, n, head_dim, chunk_tokens, s);
         if (status != KVFLUX_OK) return status;
     }
     return KVFLUX_OK;
@@ -1993,10 +2019,7 @@ int run_split(Params p, std::uint64_t rows, std::uint32_t sub, hipStream_t s) {
             if (status != KVFLUX_OK) return status;
         }
         if (p.max_chunks > 1) {
-            hipLaunchKernelGGL(paged_attention_combine_kernel,
-                               dim3(static_cast<unsigned>(n * p.query_heads)), dim3(kCombineThreads), 0, s,
-                               p, static_cast<std::uint32_t>(kD), static_cast<std::uint32_t>(kChunk));
-            const int status = launch_status("paged_attention_combine_kernel");
+            const int status = launch_combine_slice(p, n, kD, kChunk, s);
             if (status != KVFLUX_OK) return status;
         }
     }
@@ -2094,7 +2117,7 @@ int run_bs16(Params p, const Plan& plan, hipStream_t s) {
     default: status = launch_bs16<E, kD, 16>(p, plan, s); break;
     }
     if (status != KVFLUX_OK) return status;
-    if (p.max_chunks > 1) return launch_combine(p, kD, 0, s);
+    if (p.max_chunks > 1) return launch_combine(p, kD, plan.item_max > plan.item ? 0 : plan.item, s);
     return KVFLUX_OK;
 }
 

@@ -56,6 +56,11 @@ CASES = [
     ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(256)]),
     ("BFloat16", 1, 2, 64, 16, [1 + 7 * i % 1400 for i in range(257)]),
     ("Float32", 1, 1, 96, 16, [40000, 511, 512, 513]),  # the split kernel's partials, more than 64 of them
+    # More than 2048 (row, head) pairs to combine, most of them without partials.
+    ("BFloat16", 1, 16, 64, 16, [1 + 13 * i % 300 for i in range(200)] + [5000, 513, 0]),
+    ("Float16", 1, 12, 128, 16, [1 + 13 * i % 300 for i in range(300)] + [9000, 0]),  # a fixed item size
+    ("BFloat16", 1, 24, 80, 16, [1 + 13 * i % 300 for i in range(100)] + [40000, 512, 513]),
+    ("Float16", 2, 20, 256, 32, [1 + 13 * i % 300 for i in range(110)] + [36000]),
 ]
 
 
