@@ -719,8 +719,19 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
         __syncthreads();
         const std::uint32_t c = tid % kItemSizes, size = p.item_tokens + kItemStep * c;
         std::uint32_t n = 0;
+        // ceil(len / size) as the steps of the row over the candidate's steps k,
+        // by a multiplication: floor(x / k) is the high word of x * (2^32 / k
+        // rounded up) for x < 2^25 and k <= 64 (what that exceeds x / k by, at most
+        // x / 2^32, is below 1 / k; k = 1, whose factor does not fit, takes x
+        // itself). With a division for each row and candidate 250 rows of U[1, 700]
+        // tokens, 64/8 heads, took 91.8 us, now 90.7; 250 of U[1, 3000], 32/8, 294
+        // and 291.
+        const std::uint32_t steps = size / kItemStep, factor = 0xffffffffu / steps + 1;
         if (size <= p.item_max)
-            for (std::uint32_t r = tid / kItemSizes; r < rows; r += kThreads / kItemSizes) n += chunks_of(lens[r], size);
+            for (std::uint32_t r = tid / kItemSizes; r < rows; r += kThreads / kItemSizes) {
+                const std::uint32_t x = (lens[r] - (lens[r] != 0 ? 1u : 0u)) / kItemStep;
+                n += (steps == 1 ? x : __umulhi(x, factor)) + 1;
+            }
         atomicAdd(&scan[c], n);
         __syncthreads();
         const std::uint32_t walk = (scan[c] * p.heads * p.q_sets + gridDim.x - 1) / gridDim.x;
