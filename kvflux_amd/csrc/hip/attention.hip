@@ -711,8 +711,12 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
     // one lane each). Where the host allows a range, every workgroup takes
     // the size that makes the longest walk of the persistent grid shortest:
     // ceil(items / workgroups) items of that many tokens, each with the time
-    // of kItemCost more for its start and epilogue. Lane c of a wavefront
-    // weighs candidate c, its rows split over the workgroup.
+    // of kItemCost more for its start and epilogue. Of two such sizes the larger
+    // (fewer epilogues: 24 rows of 269 to 8609 tokens, 40/8 heads of 256, five walks
+    // of 768 tokens 166 us, seven of 512 174), unless it is one walk, which leaves
+    // workgroups without an item (22 rows of 2071 tokens, 40/8 heads, FP32: 352
+    // items of 1152 tokens 83.4 us, 880 of 512 79.0). Lane c of a wavefront weighs
+    // candidate c, its rows split over the workgroup.
     std::uint32_t chunk_tokens = p.item_tokens;
     if (p.item_max > p.item_tokens) {  // uniform
         if (tid < kItemSizes) scan[tid] = 0;
@@ -736,6 +740,7 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
         __syncthreads();
         const std::uint32_t walk = (scan[c] * p.heads * p.q_sets + gridDim.x - 1) / gridDim.x;
         float cost = size <= p.item_max ? static_cast<float>(walk) * static_cast<float>(size + kItemCost) : INFINITY;
+        if (walk == 1) cost += 0.5f;
         std::uint32_t best = size;
 #pragma unroll
         for (int x = 1; x < kItemSizes; x <<= 1) {
