@@ -542,8 +542,8 @@ def setup_f32(blocks, kv_heads, bs, head_size, kv_len, seed):
 
 @pytest.mark.parametrize("kv_heads,q_heads,head_size,bs,kv_len,q_tokens", F32_CASES)
 def test_prefill_f32_matches_reference(gpu, kv_heads, q_heads, head_size, bs, kv_len, q_tokens):
-    """FP32 caches on the MFMA prefill (FP32 MFMAs on Q, K, V and the weights
-    as they are, FP32 row sums): the whole output within the reference's 1e-5
+    """FP32 caches on the MFMA prefill (Q, K, V and the weights in three BF16
+    parts each, FP32 row sums): the whole output within the reference's 1e-5
     of the oracle through all three single-sequence entry points, with and
     without key splits; the split and exact entries give the same bits."""
     blocks = (kv_len + bs - 1) // bs + 17
