@@ -978,7 +978,7 @@ def bench_prefill(v2, args, stream):
                       "max_abs_err_vs_oracle": err_exact, "tolerance": 1e-5},
             # FP32 caches (the same values): one batch launch on
             # the three-part BF16 kernel, beside the FP32 MFMA peak.
-            "f32": {"kernel": "paged_prefill_kernel<f32,128> (group 4), one batch launch", "ms": f32_ms,
+            "f32": {"kernel": "paged_prefill_f32_kernel<128> (group 4), one batch launch", "ms": f32_ms,
                     "TFLOPs": flops / (f32_ms * 1e-3) / 1e12,
                     "frac_of_fp32_mfma_peak": flops / (f32_ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS,
                     "max_abs_err_vs_oracle": err_f32, "tolerance": 1e-5},

@@ -227,8 +227,9 @@ int kvflux_paged_attention_noalloc(const void* key_cache, const void* value_cach
  * query i attends to tokens [0, kv_len - query_tokens + i].
  * F16/BF16 caches: Q is rounded to the cache dtype and the softmax weights to
  * the cache dtype before the MFMA products; accumulation and softmax are
- * FP32. F32 caches: Q, K, V and the weights as three BF16 parts each (FP32
- * accuracy; FP32 MFMAs where a value has no such parts: the 1e-5 contract of kvflux_paged_prefill_exact, head_size 64 or 128).
+ * FP32. F32 caches: Q, K, V and the weights as three BF16 parts each, with
+ * FP32 MFMAs where a value has no such parts (2^56 and more, under 2^-100): the
+ * 1e-5 contract of kvflux_paged_prefill_exact, head_size 64 or 128.
  * KVFLUX_ERR_UNSUPPORTED unless head_size is 64, 128 or 256 (F32: 64 or
  * 128), block_size is a power of two up to 256 and kv_len is below 2^31.
  * Any GQA group query_heads / num_kv_heads: up to 512 at head_size 64, 256 at
@@ -276,7 +277,8 @@ int kvflux_paged_prefill_split(const void* key_cache, const void* value_cache,
  * folded in) and the softmax weights enter the MFMAs as three 16-bit parts
  * each, so every product is exact in FP32, and the row sums are FP32 sums of
  * the weights. About three times the MFMA work of kvflux_paged_prefill_split.
- * F32 caches run the FP32-MFMA prefill, as in kvflux_paged_prefill_split.
+ * F32 caches run the same kernel as in kvflux_paged_prefill_split (K and V in
+ * three parts as well).
  * Same arguments, workspace and errors, except that head_size must be 64 or
  * 128 (256: KVFLUX_ERR_UNSUPPORTED). Replaces paged_attention_kernel
  * (reference src/v2/paged_attention.cu:108-128, 193-246) for the

@@ -1301,7 +1301,7 @@ int launch_prefill_head_size(const PrefillParams& p, std::uint64_t head_size, st
 struct PrefillPlan {
     std::uint32_t splits;       // key splits per (query block, kv head)
     std::uint32_t split_tiles;  // 64-key tiles per split
-    std::uint64_t workspace;    // bytes of partials (0 when splits == 1)
+    std::uint64_t workspace;    // prefill_most_splits: bytes of partials (0 when splits == 1)
     int key_parts;              // 2: the wavefronts of a workgroup split the keys (kKs)
 };
 
@@ -1328,7 +1328,8 @@ inline PrefillPlan prefill_most_splits(std::uint64_t head_size, std::uint64_t gr
 }
 
 // Key splits (1 .. most_splits) and key parts (1 or 2) of a launch: the pair
-// with the shortest estimated time on 256 CUs of one resident workgroup each.
+// with the shortest estimated time on an MI355X's 256 CUs, of one resident
+// workgroup each (a partition of fewer takes the same plans).
 // A workgroup takes kStart (mostly its FP32 query rows and outputs on their
 // way through memory: 256 workgroups of 64 tokens x 4 heads and one tile take
 // 17 us), then per tile the time of its MFMAs (halved with two key parts) and
@@ -1349,7 +1350,8 @@ inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32,
                                   std::uint64_t num_kv_heads, std::uint64_t kv_len, std::uint64_t query_tokens,
                                   std::uint64_t query_heads, std::uint64_t most_splits, bool key_parts_allowed) {
     constexpr double kCus = 256, kStart = 10.0, kStep = 0.35, kBytesPerUs = 5e6;
-    // us of a tile's MFMAs in a workgroup, from 8 x 4096 tokens
+    // us of a tile's MFMAs in a workgroup, from 8 x 4096 tokens (FP32: with kStep
+    // 5.35 of the 5.6 measured; its loads and conversions run under them)
     const double mfma = (f32 ? 5.0 : exact ? 2.5 : 1.7) * (f32 || exact ? head_size / 128.0 : 1.0);
     const double margin = exact ? 1.25 : 1.05;
     const std::uint64_t tiles = (kv_len + kPfTile - 1) / kPfTile;
@@ -1386,8 +1388,6 @@ inline PrefillPlan prefill_choice(std::uint64_t head_size, bool exact, bool f32,
             }
         }
     }
-    if (best.splits > 1)
-        best.workspace = best.splits * query_tokens * query_heads * (head_size + 2) * sizeof(float);
     return best;
 }
 
@@ -1422,7 +1422,7 @@ int paged_prefill(const void* key_cache, const void* value_cache, uint64_t num_b
         num_kv_heads * block_size * head_size * dtype_bytes(dtype) > 0xffffffffULL) {
         return fail(KVFLUX_ERR_UNSUPPORTED, "paged prefill: shape not handled by the MFMA kernel");
     }
-    // FP32 caches always take the FP32 MFMAs, whose products are exact.
+    // FP32 caches have one variant, of FP32 accuracy.
     if (dtype == KVFLUX_DTYPE_F32) exact = true;
     if (exact && head_size == 256) return fail(KVFLUX_ERR_UNSUPPORTED, "exact paged prefill: head_size 256");
 
