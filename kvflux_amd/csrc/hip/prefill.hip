@@ -829,9 +829,9 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 // Measured against v_mfma_f32_16x16x4_f32 throughout, 64-bit errors beside:
 // 4 x 384..1024 tokens, 16/4 heads 132.3 -> 93.4 us (3.3e-7 -> 2.0e-7), 813
 // tokens, 12/1 heads 63.8 -> 45.6 (4.0e-7 -> 2.5e-7), 8 x 4096 tokens, 32/8
-// heads 8874 -> 6411 us (3.7e-7 -> 2.4e-7). What bounds it now is LDS reads
-// (384 KiB per half and workgroup, 128 bytes a clock: 1.3 of 2.8 us) beside
-// 96 MFMAs per wavefront and half (1.3 us).
+// heads 8874 -> 6083 us (3.7e-7 -> 2.4e-7). What bounds it now is a wavefront's
+// chain: counters show the MFMAs busy 44 %, LDS 29 % without conflicts, and a
+// wavefront waiting 31 % of its time for operands and 31 % for a busy unit.
 template <int kD>
 __global__ __launch_bounds__(kPfThreads) void paged_prefill_f32_kernel(PrefillParams p) {
     using M = PfBf16Exact;
