@@ -825,7 +825,8 @@ __global__ __launch_bounds__(kPfThreads) void paged_prefill_kernel(PrefillParams
 //    products drop).
 //  * A half with a value without parts, and every half of a wavefront with
 //    such a query row, takes the FP32 MFMAs on values read from global memory
-//    (direct_scores, direct_values).
+//    (direct_scores, direct_values): about twelve times as slow, for inputs that
+//    are hardly met (every half so, 4 x 384..1024 tokens: 1.19 ms).
 // Measured against v_mfma_f32_16x16x4_f32 throughout, 64-bit errors beside:
 // 4 x 384..1024 tokens, 16/4 heads 132.3 -> 93.4 us (3.3e-7 -> 2.0e-7), 813
 // tokens, 12/1 heads 63.8 -> 45.6 (4.0e-7 -> 2.5e-7), 8 x 4096 tokens, 32/8

@@ -1,4 +1,5 @@
-"""Work-item sizes of the block-size-16 decode kernel, chosen on the device
+"""Plans of the block-size-16 decode kernel: short rows in one launch, head sets
+and their rest, and work-item sizes, chosen on the device
 from the row lengths: rows around multiples of the 128-token step, launches of
 one row up to one past the largest that chooses, empty rows, pages whose
 slots bound the item, a workspace of the least size (512-token items) beside
