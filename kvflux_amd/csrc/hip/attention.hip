@@ -186,6 +186,7 @@ struct Params {
     // item_tokens to item_max.
     std::uint32_t item_tokens;
     std::uint32_t item_max;
+    std::uint32_t at_once;  // items that run about as fast as one alone, for that choice
     // Block-size-16 kernel: query heads per kv head (the GQA group), the
     // first of them a launch serves (0), and the head sets of a group above 8
     // (group / sub-group, each a work item of its own; 1 otherwise).
@@ -710,8 +711,9 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
     // wavefront, at most 64, whose page offsets (small pages: page slots) fit
     // one lane each). Where the host allows a range, every workgroup takes
     // the size that makes the longest walk of the persistent grid shortest:
-    // ceil(items / workgroups) items of that many tokens, each with the time
-    // of kItemCost more for its start and epilogue. Of two such sizes the larger
+    // ceil(items / workgroups) items of that many tokens (small calls: items over
+    // CUs, Params::at_once), each with the time of kItemCost more for its start
+    // and epilogue. Of two such sizes the larger
     // (fewer epilogues: 24 rows of 269 to 8609 tokens, 40/8 heads of 256, five walks
     // of 768 tokens 166 us, seven of 512 174), unless it is one walk, which leaves
     // workgroups without an item (22 rows of 2071 tokens, 40/8 heads, FP32: 352
@@ -738,7 +740,8 @@ __global__ __launch_bounds__(kThreads, (bs16_occupancy_g<E, kD, kG, kSmall>())) 
             }
         atomicAdd(&scan[c], n);
         __syncthreads();
-        const std::uint32_t walk = (scan[c] * p.heads * p.q_sets + gridDim.x - 1) / gridDim.x;
+        const std::uint32_t at_once = gridDim.x < p.at_once ? gridDim.x : p.at_once;
+        const std::uint32_t walk = (scan[c] * p.heads * p.q_sets + at_once - 1) / at_once;
         float cost = size <= p.item_max ? static_cast<float>(walk) * static_cast<float>(size + kItemCost) : INFINITY;
         if (walk == 1) cost += 0.5f;
         std::uint32_t best = size;
@@ -1661,30 +1664,42 @@ __global__ __launch_bounds__(64) void paged_attention_generic_kernel(Params p, s
 // once per (kernel, device). Devices past kMaxDevices are queried per call.
 constexpr int kMaxDevices = 64;
 
+// at_once: two items on a CU take nearly twice the time of one, so small calls
+// count their walks in CUs (1 row of 25164 tokens, 28/4 heads of 64: 640 items of
+// 128 tokens 22.8 us, 320 of 256 18.8, 160 of 512 18.1; 1 of 16000, 32/8 heads of
+// 128, FP32: 504 of 256 36.9, 256 of 512 33.0; 1 of 12171, 16/4 heads of 64: 192 of
+// 256 15.6). Workgroups of small pages wait on their gathered rows and share a CU
+// well (8-token pages, head size 64: 3 rows of 2093 to 16751 tokens, 8/8 heads,
+// 736 of 256 20.4, 246 of 768 22.1; 24 rows of 500 to 12000, 14/1 heads 20.9, by
+// CUs 25.3).
+struct Resident {
+    int slots = 0;    // workgroups the device holds: CUs x occupancy
+    int at_once = 0;  // of them, those that run about as fast as one alone
+};
+
 template <typename E, int kD, int kG, bool kSmall>
-int resident_slots(int* out) {
-    static std::atomic<int> cache[kMaxDevices];
+int resident_slots(Resident* out) {
+    static std::atomic<std::uint64_t> cache[kMaxDevices];  // CUs, occupancy
     int device = 0;
     int status = hip_status(hipGetDevice(&device), "hipGetDevice");
     if (status != KVFLUX_OK) return status;
-    if (device >= 0 && device < kMaxDevices) {
-        const int known = cache[device].load(std::memory_order_relaxed);
-        if (known > 0) {
-            *out = known;
-            return KVFLUX_OK;
-        }
+    const bool cached = device >= 0 && device < kMaxDevices;
+    std::uint64_t known = cached ? cache[device].load(std::memory_order_relaxed) : 0;
+    if (known == 0) {
+        int cus = 0, per_cu = 0;
+        status = hip_status(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device),
+                            "hipDeviceGetAttribute");
+        if (status == KVFLUX_OK)
+            status = hip_status(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                                    &per_cu, paged_decode_bs16_kernel<E, kD, kG, kSmall>, kThreads, 0),
+                                "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+        if (status != KVFLUX_OK) return status;
+        known = static_cast<std::uint64_t>(cus > 0 ? cus : 1) << 32 | static_cast<std::uint32_t>(per_cu > 0 ? per_cu : 1);
+        if (cached) cache[device].store(known, std::memory_order_relaxed);
     }
-    int cus = 0, per_cu = 0;
-    status = hip_status(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device),
-                        "hipDeviceGetAttribute");
-    if (status == KVFLUX_OK)
-        status = hip_status(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                &per_cu, paged_decode_bs16_kernel<E, kD, kG, kSmall>, kThreads, 0),
-                            "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-    if (status != KVFLUX_OK) return status;
-    const int slots = (cus > 0 ? cus : 1) * (per_cu > 0 ? per_cu : 1);
-    if (device >= 0 && device < kMaxDevices) cache[device].store(slots, std::memory_order_relaxed);
-    *out = slots;
+    const int cus = static_cast<int>(known >> 32), per_cu = static_cast<int>(known & 0xffffffffu);
+    out->slots = cus * per_cu;
+    out->at_once = kSmall ? cus * per_cu : cus;
     return KVFLUX_OK;
 }
 
@@ -1698,12 +1713,13 @@ struct Plan {
     std::uint32_t item_max = kChunk;  // Bs16: above it, the kernel chooses up to this many
     unsigned grid = 0;         // Bs16: persistent grid
     std::uint64_t chunks = 0;  // partial slots per (row, query head); <= 1: no partials
+    std::uint32_t at_once = 1, rest_at_once = 1;  // Bs16: Params::at_once of the launches
     std::uint32_t rest = 0;    // Bs16: heads past the last whole set (a second launch), 0 if none
     unsigned rest_grid = 0;    // Bs16: persistent grid of that launch
 };
 
 template <typename E, int kD, bool kSmall>
-int resident_slots_for(std::uint32_t sub, int* out) {
+int resident_slots_for(std::uint32_t sub, Resident* out) {
     switch (sub) {
     case 1: return resident_slots<E, kD, 1, kSmall>(out);
     case 2: return resident_slots<E, kD, 2, kSmall>(out);
@@ -1735,7 +1751,7 @@ int resident_slots_for(std::uint32_t sub, int* out) {
 
 // Resident workgroups of the block-size-16 kernel on items of `sub` heads.
 template <typename E, int kD>
-int bs16_slots(bool small, std::uint32_t sub, int* out) {
+int bs16_slots(bool small, std::uint32_t sub, Resident* out) {
     return small ? resident_slots_for<E, kD, true>(sub, out) : resident_slots_for<E, kD, false>(sub, out);
 }
 
@@ -1869,7 +1885,7 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             // 8, say) takes sets of 16 (or 8) heads plus one launch for the
             // heads past the last set, rather than many narrow sets.
             std::uint32_t rest = 0;
-            int rest_slots = 0;
+            Resident others;  // of the launch for the rest
             if (!small && kD != 256 && g > 8 && sub < 4) {
                 sub = g > 16 && g % 16 <= 8 ? 16u : 8u;
                 rest = g % sub;
@@ -1885,24 +1901,25 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
                 // more rounds of 512-token items than two (4 rows of 300 to 2000
                 // tokens, 1 kv head, group 11, 64, 128 and 256: 15.2 and 20.1,
                 // 18.7 and 22.6, 22.5 and 27.8 us).
-                int narrow = 0, wide = 0;
+                Resident narrow, wide;
                 int st = bs16_slots<E, kD>(small, sub, &narrow);
                 if (st == KVFLUX_OK) st = bs16_slots<E, kD>(small, cap, &wide);
-                if (st == KVFLUX_OK) st = bs16_slots<E, kD>(small, g % cap, &rest_slots);
+                if (st == KVFLUX_OK) st = bs16_slots<E, kD>(small, g % cap, &others);
                 if (st != KVFLUX_OK) return st;
                 const std::uint64_t items = rows * max_chunks * p.heads;
-                auto rounds = [](std::uint64_t n, int slots) { return (n + slots - 1) / slots; };
-                if (rounds(items * (g / sub), narrow) > rounds(items * (g / cap), wide) + rounds(items, rest_slots)) {
+                auto rounds = [](std::uint64_t n, const Resident& r) { return (n + r.slots - 1) / r.slots; };
+                if (rounds(items * (g / sub), narrow) > rounds(items * (g / cap), wide) + rounds(items, others)) {
                     sub = cap;
                     rest = g % sub;
                 }
             }
             const std::uint64_t sets = g / sub;  // head sets per kv head, each its own work items
             if (2 * rows * max_chunks * p.heads * sets > 0xffffffffULL) return plan_fallback(kD, group, max_chunks, plan);
-            int slots = 0;
-            int status = bs16_slots<E, kD>(small, sub, &slots);
-            if (status == KVFLUX_OK && rest > 0) status = bs16_slots<E, kD>(small, rest, &rest_slots);
+            Resident resident;
+            int status = bs16_slots<E, kD>(small, sub, &resident);
+            if (status == KVFLUX_OK && rest > 0) status = bs16_slots<E, kD>(small, rest, &others);
             if (status != KVFLUX_OK) return status;
+            const int slots = resident.slots, rest_slots = others.slots;
             // Work item size: the largest chunk (up to 4096 tokens, less for
             // small pages) that still gives at least 8 items per resident
             // workgroup when every row is kv_len long.
@@ -1925,13 +1942,14 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             const std::uint64_t fine = fine_items(rows, p.kv_len, p.heads, p.query_heads, bs, kD);
             if (fine > 0 && scratch_bytes >= fine && kFineItem < item) {
                 const std::uint64_t per_row = rows * p.heads, parts = (p.kv_len + kFineItem - 1) / kFineItem;
-                auto rounds = [&](std::uint64_t n) {
-                    return (per_row * sets * n + slots - 1) / slots +
-                           (rest > 0 ? (per_row * n + rest_slots - 1) / rest_slots : 0);
+                auto rounds = [&](std::uint64_t n, std::uint64_t at_once, std::uint64_t rest_at_once) {
+                    return (per_row * sets * n + at_once - 1) / at_once +
+                           (rest > 0 ? (per_row * n + rest_at_once - 1) / rest_at_once : 0);
                 };
                 const double combine = combine_tokens(kD, kF32Cache, small) * (1.0 + per_row * sets * parts / 1024.0);
-                if (!whole_rows || static_cast<double>(rounds(1) * (whole + kItemCost)) >
-                                       static_cast<double>(rounds(parts) * (kFineItem + kItemCost)) + combine) {
+                if (!whole_rows || static_cast<double>(rounds(1, slots, rest_slots) * (whole + kItemCost)) >
+                                       static_cast<double>(rounds(parts, resident.at_once, others.at_once) * (kFineItem + kItemCost)) +
+                                           combine) {
                     item = kFineItem;
                     whole_rows = false;
                 }
@@ -1945,6 +1963,8 @@ int plan_group(const Params& p, std::uint64_t rows, std::uint64_t group, std::ui
             plan->small = small;
             plan->item = item;
             plan->item_max = item_max;
+            plan->at_once = static_cast<std::uint32_t>(item == kFineItem ? resident.at_once : slots);
+            plan->rest_at_once = static_cast<std::uint32_t>(item == kFineItem ? others.at_once : rest_slots);
             plan->grid = static_cast<unsigned>(items == 0 ? 1 : items < static_cast<std::uint64_t>(slots) ? items : slots);
             plan->chunks = chunks;
             plan->rest = rest;
@@ -2095,6 +2115,7 @@ int run_bs16(Params p, const Plan& plan, hipStream_t s) {
     p.bs_shift = log2_pow2(bs);
     p.item_tokens = plan.item;
     p.item_max = plan.item_max;
+    p.at_once = plan.at_once;
     // One launch: a group above 8 is served as head sets of the sub-group,
     // each a work item of its own (and the heads past the last whole set, if
     // any, by a second launch).
@@ -2106,6 +2127,7 @@ int run_bs16(Params p, const Plan& plan, hipStream_t s) {
         r.q_first = plan.sub * p.q_sets;
         r.q_sets = 1;
         Plan rp = plan;
+        r.at_once = plan.rest_at_once;
         rp.grid = plan.rest_grid;
         switch (plan.rest) {
         case 1: status = launch_bs16<E, kD, 1>(r, rp, s); break;
